@@ -282,3 +282,13 @@ def load_library():
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+def by_address(name):
+    """The library function `name` with every argument passed as a plain address (an int, a c_void_p or None): what the
+    enqueue calls use, because building a typed pointer per argument costs more than the C side of such a call."""
+    fn = load_library()[name]  # (a function object of its own: indexing does not share it with the attribute)
+    res, args = SYMBOLS[name]
+    fn.restype = res
+    fn.argtypes = [C.c_void_p] * len(args)
+    return fn

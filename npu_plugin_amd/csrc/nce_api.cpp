@@ -6,6 +6,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <atomic>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -17,6 +18,9 @@
 
 struct nce_executor_s {
     int device = 0;
+    // Never used twice in a process (an executor's address can be): what kept launches of single tasks belong to.
+    const uint64_t id = next_id.fetch_add(1);
+    static std::atomic<uint64_t> next_id;
     nce_log_s* log = nullptr;
     nce::Options opt;  // tuning knobs, read from the environment once at creation
     // Persistent segments: a pinned host word their kernels raise when a bounded wait ran out (checked after a
@@ -45,6 +49,7 @@ struct nce_executor_s {
 };
 
 thread_local nce::LaunchContext nce::tls_launch;
+std::atomic<uint64_t> nce_executor_s::next_id{1};
 
 namespace {
 // Launches of the fixed workspace that gave up, per device and process (see nce_executor_s::ws_failures_seen).
@@ -500,6 +505,54 @@ nce_result_t launch_plan(nce_executor_s* ex, const Plan& plan, hipStream_t strea
     return NCE_RESULT_SUCCESS;
 }
 
+// ---- kept launches of single tasks -----------------------------------------------------------------------------------------
+// A program enqueues the same few descriptors over and over. Validating one and working out its kernel, grid and argument
+// block costs about as much host time as a tenth to a quarter of the launch itself, and for small tasks the host is what the
+// GPU waits for: so every host thread keeps the prepared launches of the descriptors it enqueued last. An entry holds a
+// copy of everything the launches were made from - the descriptor, its variant and its PPE task, compared byte by byte on
+// every call - and is used only if nothing of it changed; tensors are read by the kernels, never by the host, so their
+// contents do not matter. Descriptors of more than one variant, executors that log kernel choices and tasks whose planning
+// logged a warning (it is due on every call) are planned anew each time.
+struct KeptTask {
+    uint64_t executor = 0;  // 0: empty
+    nce_cluster_task_desc_t desc;
+    nce_dpu_task_t variant;
+    nce_ppe_task_t ppe;
+    std::vector<nce::RecordedLaunch> launches;
+
+    bool holds(uint64_t ex, const nce_cluster_task_desc_t* t) const {
+        return executor == ex && memcmp(&desc, t, sizeof(desc)) == 0 && memcmp(&variant, t->variants, sizeof(variant)) == 0 &&
+               (t->ppe == nullptr || memcmp(&ppe, t->ppe, sizeof(ppe)) == 0);
+    }
+    void keep(uint64_t ex, const nce_cluster_task_desc_t* t, std::vector<nce::RecordedLaunch>&& l) {
+        memcpy(&desc, t, sizeof(desc));
+        memcpy(&variant, t->variants, sizeof(variant));
+        if (t->ppe != nullptr) memcpy(&ppe, t->ppe, sizeof(ppe));
+        launches = std::move(l);
+        executor = ex;
+    }
+};
+constexpr int kKeptTasks = 64;  // per thread, by the descriptor's address: 64 x 0.7 KiB and the launches' argument blocks
+thread_local std::unique_ptr<KeptTask[]> tls_kept;
+
+KeptTask* kept_slot(const nce_cluster_task_desc_t* t) {
+    if (!tls_kept) tls_kept.reset(new KeptTask[kKeptTasks]);
+    const uint64_t h = reinterpret_cast<uintptr_t>(t) * 0x9E3779B97F4A7C15ull;
+    return &tls_kept[h >> (64 - 6)];
+}
+
+nce_result_t replay_all(nce_executor_s* ex, const std::vector<nce::RecordedLaunch>& launches, hipStream_t stream) {
+    for (const nce::RecordedLaunch& l : launches) {
+        const hipError_t e = nce::replay(l, stream);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            ex->log->add(1, "kernel launch failed: %s", hipGetErrorString(e));
+            return NCE_RESULT_ERROR_UNKNOWN;
+        }
+    }
+    return NCE_RESULT_SUCCESS;
+}
+
 }  // namespace
 
 // A task list keeps the validated plans and, from its first Enqueue on, the prepared launches (kernel, grid and
@@ -801,7 +854,15 @@ nce_result_t nceClusterTaskValidate(nce_executor_handle_t executor, const nce_cl
 nce_result_t nceClusterTaskEnqueue(nce_executor_handle_t executor, const nce_cluster_task_desc_t* task, void* hip_stream) {
     if (executor == nullptr) return NCE_RESULT_ERROR_INVALID_NULL_HANDLE;
     try {
+        const hipStream_t stream = static_cast<hipStream_t>(hip_stream);
+        const bool keepable = task != nullptr && task->num_variants == 1 && task->variants != nullptr && executor->log->level < 3 && executor->device >= 0;
+        KeptTask* const kept = keepable ? kept_slot(task) : nullptr;
+        if (kept != nullptr && kept->holds(executor->id, task)) {
+            if (hipSetDevice(executor->device) != hipSuccess) return NCE_RESULT_ERROR_UNKNOWN;
+            return replay_all(executor, kept->launches, stream);
+        }
         Plan plan;
+        const uint64_t lines = executor->log->lines.load(std::memory_order_relaxed);
         const nce_result_t r = make_plan(executor->log, task, &plan);
         if (r != NCE_RESULT_SUCCESS) return r;
         if (executor->device < 0) {
@@ -809,8 +870,18 @@ nce_result_t nceClusterTaskEnqueue(nce_executor_handle_t executor, const nce_clu
             return NCE_RESULT_ERROR_UNSUPPORTED;
         }
         if (hipSetDevice(executor->device) != hipSuccess) return NCE_RESULT_ERROR_UNKNOWN;
-        const ScopedLaunch ctx(&executor->opt, nullptr, executor->log);
-        return launch_plan(executor, plan, static_cast<hipStream_t>(hip_stream));
+        if (kept == nullptr || executor->log->lines.load(std::memory_order_relaxed) != lines) {
+            const ScopedLaunch ctx(&executor->opt, nullptr, executor->log);
+            return launch_plan(executor, plan, stream);
+        }
+        std::vector<nce::RecordedLaunch> launches;
+        {
+            const ScopedLaunch ctx(&executor->opt, &launches, executor->log);
+            const nce_result_t q = launch_plan(executor, plan, stream);
+            if (q != NCE_RESULT_SUCCESS) return q;
+        }
+        kept->keep(executor->id, task, std::move(launches));
+        return replay_all(executor, kept->launches, stream);
     } catch (const std::bad_alloc&) {
         return NCE_RESULT_ERROR_OUT_OF_MEMORY;
     } catch (...) {
@@ -922,14 +993,7 @@ nce_result_t enqueue_list(nce_task_list_handle_t list, void* hip_stream, bool fi
             }
             ex->ws_used.store(true);
         }
-        for (const nce::RecordedLaunch& l : list->launches) {
-            const hipError_t e = nce::replay(l, stream);
-            if (e != hipSuccess) {
-                ex->log->add(1, "kernel launch failed: %s", hipGetErrorString(e));
-                return NCE_RESULT_ERROR_UNKNOWN;
-            }
-        }
-        return NCE_RESULT_SUCCESS;
+        return replay_all(ex, list->launches, stream);
     } catch (const std::bad_alloc&) {
         return NCE_RESULT_ERROR_OUT_OF_MEMORY;
     } catch (...) {

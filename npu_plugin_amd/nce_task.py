@@ -106,6 +106,7 @@ class NCEClusterTask:
         self.desc.kernel_pad_top, self.desc.kernel_pad_bottom = top, bottom
         self._variants = []
         self._ppe = None
+        self._wired = (None, None, None)  # (descriptor, variant, PPE task) that finalize() has connected
 
     def addDPUTask(self, outStart, outEnd, pad=(0, 0, 0, 0), mpeMode=abi.MPE_CUBOID_16x16, clusterId=0):
         """outStart / outEnd: [x, y, z] inclusive; pad: (left, right, top, bottom)
@@ -153,18 +154,30 @@ class NCEClusterTask:
 
     def finalize(self):
         """Materialise the variant array and PPE pointer; returns the ctypes descriptor."""
-        n = len(self._variants)
-        self._variant_array = (abi.DpuTask * max(n, 1))(*self._variants)
-        self.desc.variants = C.cast(self._variant_array, C.POINTER(abi.DpuTask)) if n else None
-        self.desc.num_variants = n
-        self.desc.ppe = C.pointer(self._ppe) if self._ppe is not None else None
-        return self.desc
+        variants, desc, ppe = self._variants, self.desc, self._ppe
+        n = len(variants)
+        if n == 1:
+            # The usual case, one variant: the descriptor points at the DpuTask and PpeTask structs themselves, so later
+            # changes to their fields are seen and nothing has to be built again for the next call.
+            wired = self._wired
+            if wired[0] is desc and wired[1] is variants[0] and wired[2] is ppe and desc.num_variants == 1:
+                return desc
+            desc.variants = C.pointer(variants[0])
+            self._wired = (desc, variants[0], ppe)
+        else:
+            self._variant_array = (abi.DpuTask * max(n, 1))(*variants)
+            desc.variants = C.cast(self._variant_array, C.POINTER(abi.DpuTask)) if n else None
+            self._wired = (None, None, None)
+        desc.num_variants = n
+        desc.ppe = C.pointer(ppe) if ppe is not None else None
+        return desc
 
 
 class TaskList:
     def __init__(self, executor):
         self._ex = executor
         self._lib = executor._lib
+        self._list_enqueue = abi.by_address("nceTaskListEnqueue")
         self._h = C.c_void_p()
         executor._check(self._lib.nceTaskListCreate(executor._h, C.byref(self._h)))
         self._keep = []
@@ -174,7 +187,9 @@ class TaskList:
         self._ex._check(self._lib.nceTaskListAppend(self._h, C.byref(task.finalize())))
 
     def enqueue(self, stream=None):
-        self._ex._check(self._lib.nceTaskListEnqueue(self._h, C.c_void_p(stream or 0)))
+        rc = self._list_enqueue(self._h, stream)
+        if rc != abi.SUCCESS:
+            self._ex._check(rc)
 
     def enqueue_no_alloc(self, stream=None):
         """nceTaskListEnqueueNoAlloc: the same launches with no device allocation (the library's fixed workspace)."""
@@ -191,6 +206,7 @@ class Executor:
 
     def __init__(self, device_id=0, log_level=2):
         self._lib = abi.load_library()
+        self._task_enqueue = abi.by_address("nceClusterTaskEnqueue")
         self._h = C.c_void_p()
         self._log = C.c_void_p()
         rc = self._lib.nceExecutorCreate(abi.ExecutorDesc(device_id, log_level), C.byref(self._h), C.byref(self._log))
@@ -215,7 +231,9 @@ class Executor:
         self._check(self.validate_code(task))
 
     def enqueue(self, task, stream=None):
-        self._check(self._lib.nceClusterTaskEnqueue(self._h, C.byref(task.finalize()), C.c_void_p(stream or 0)))
+        rc = self._task_enqueue(self._h, C.addressof(task.finalize()), stream)
+        if rc != abi.SUCCESS:
+            self._check(rc)
 
     def synchronize(self, stream=None):
         self._check(self._lib.nceExecutorSynchronize(self._h, C.c_void_p(stream or 0)))
