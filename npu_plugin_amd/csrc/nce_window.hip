@@ -373,6 +373,155 @@ __global__ __launch_bounds__(NT) void window_kernel(WinArgs a) {
     }
 }
 
+// AVEPOOL over windows without a compile-time form (the 7x7 of a global pool, 4x4, 11x11 ...): the taps of an output are
+// spread over lanes. One lane per output makes a global pool a chain of 49 loads on a twentieth of the chip (64 x 7 x 7 x 1280:
+// 80 wavefronts, 23 us for 4 MB); here a wavefront owns one output pixel of up to 8 channel groups, lane = part * G + group,
+// and its 64 / G parts take every 64 / G-th tap each (7 of 49 taps with 8 groups, all requested at once). Sums run on pairs of
+// 16-bit values (even and odd bytes of a dword; 121 taps * 255 stays below 2^16), the parts are added up by lane exchanges and
+// four of them requantise one dword of the group each. No LDS, no barrier. Bound by the latency of launch, arguments and one
+// round trip to memory at the sizes of a global pool.
+struct SplitArgs {
+    TaskDev t;
+    Box box;
+    uint32_t nitems;    // output pixels of the box x slabs (of 2^glog channel groups)
+    uint32_t nslabs;
+    int32_t glog;       // log2 of the channel groups per wavefront
+    int32_t ntaps;
+    FastDiv div_slabs, div_bw, div_bh, div_kx;
+    uint32_t a_xor, fill;
+    int32_t zpu;
+};
+
+__global__ __launch_bounds__(NT) void avgpool_split_kernel(SplitArgs a) {
+    prefetch_kernel_arguments<sizeof(SplitArgs)>();
+    const TaskDev& t = a.t;
+    const Box& box = a.box;
+    const int lane = threadIdx.x & 63;
+    const uint32_t item = blockIdx.x * (NT / 64) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (item >= a.nitems) return;  // uniform for the wavefront
+    const uint32_t r1 = fdiv(item, a.div_slabs);
+    const uint32_t slab = item - r1 * a.nslabs;
+    const uint32_t r2 = fdiv(r1, a.div_bw);
+    const int32_t ox = box.x0 + (int32_t)(r1 - r2 * (uint32_t)box.bw);
+    const uint32_t n = fdiv(r2, a.div_bh);
+    const int32_t oy = box.y0 + (int32_t)(r2 - n * (uint32_t)box.bh);
+
+    const int cgroups = box.bc >> 4;
+    const int group = (int)(slab << a.glog) + (lane & ((1 << a.glog) - 1));
+    const int part = lane >> a.glog, parts = 64 >> a.glog;
+    const int32_t oc = box.z0 + (min(group, cgroups - 1) << 4);  // (lanes past the last group read a duplicate, store nothing)
+    const int32_t iy0 = oy * t.sy - t.pt, ix0 = ox * t.sx - t.pl;
+    const uint8_t* const src = t.in.data + (int64_t)n * t.in.sn + oc;
+
+    // the table rows of this lane's four channels travel with the taps
+    const bool store = part < 4 && group < cgroups;
+    int32_t tw2[4], tbias[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        tw2[i] = tbias[i] = 0;
+        if (t.table != nullptr && store) {
+            const int32_t* const row = t.table + (int64_t)(oc + 4 * part + i) * t.table_stride;
+            tw2[i] = row[2];
+            tbias[i] = row[3];
+        }
+    }
+    uint32_t se[4] = {0, 0, 0, 0}, so[4] = {0, 0, 0, 0};  // sums of the even / odd bytes of each dword
+    constexpr int UNROLL = 8;
+    for (int t0 = part; t0 < a.ntaps; t0 += UNROLL * parts) {
+        uint4 v[UNROLL];
+        bool ok[UNROLL];
+#pragma unroll
+        for (int j = 0; j < UNROLL; ++j) {
+            const int tap = min(t0 + j * parts, a.ntaps - 1);
+            const int ky = (int)fdiv((uint32_t)tap, a.div_kx), kx = tap - ky * t.kx;
+            const int32_t iy = iy0 + ky, ix = ix0 + kx;
+            ok[j] = (uint32_t)iy < (uint32_t)t.in.h && (uint32_t)ix < (uint32_t)t.in.w;
+            const int32_t cy = min(max(iy, 0), t.in.h - 1), cx = min(max(ix, 0), t.in.w - 1);
+            v[j] = *reinterpret_cast<const uint4*>(src + (int64_t)cy * t.in.sh + (int64_t)cx * t.in.sw);
+        }
+#pragma unroll
+        for (int j = 0; j < UNROLL; ++j) {
+            const bool real = t0 + j * parts < a.ntaps;
+            const uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                const uint32_t x = real ? (ok[j] ? w[d] ^ a.a_xor : a.fill) : 0u;
+                // (no carry from the low into the high half: both sums stay below 2^16)
+                se[d] += x & 0x00FF00FFu;
+                so[d] += (x >> 8) & 0x00FF00FFu;
+            }
+        }
+    }
+    for (int m = 1 << a.glog; m < 64; m <<= 1) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            se[d] += (uint32_t)__shfl_xor((int)se[d], m);
+            so[d] += (uint32_t)__shfl_xor((int)so[d], m);
+        }
+    }
+    // dword `part` of the group: channels 4 * part .. + 3
+    const uint32_t e = part == 0 ? se[0] : part == 1 ? se[1] : part == 2 ? se[2] : se[3];
+    const uint32_t o = part == 0 ? so[0] : part == 1 ? so[1] : part == 2 ? so[2] : so[3];
+    const int32_t sum[4] = {(int32_t)(e & 0xFFFFu), (int32_t)(o & 0xFFFFu), (int32_t)(e >> 16), (int32_t)(o >> 16)};
+    const int32_t corr = -a.zpu * a.ntaps;  // out-of-image taps entered with the zero point
+    int32_t mult[4], shift[4];
+    bool bad = false, sat = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        mult[i] = t.table != nullptr ? table_mult(tw2[i]) : t.ppe.quant_mult;
+        shift[i] = t.table != nullptr ? table_shift(tw2[i]) : t.ppe.quant_shift;
+        bad = bad || (store && shift[i] > kMaxF64Shift);
+        sat = sat || (store && ppe_may_saturate((int64_t)a.ntaps * 255, tbias[i], mult[i], shift[i]));
+    }
+    const PpeF64 pu = ppe_f64_setup(t.ppe, __any(sat));
+    const int pmode = ppe_mode_of(pu, __any(bad));
+    uint32_t packed = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        int32_t y;
+        if (pmode == PPE_MODE_INT) {
+            y = ppe_apply(sum[i] + corr, tbias[i], mult[i], shift[i], t.ppe);
+        } else {
+            const double M = ppe_scale_M(mult[i], shift[i]);
+            const double v = __builtin_fma((double)(sum[i] + corr), M, ppe_mode_B(ppe_scale_B(tbias[i], M, shift[i], t.ppe.round_mode), pmode, pu));
+            y = pmode == PPE_MODE_FOLDED ? ppe_finish_mode<PPE_MODE_FOLDED>(v, pu) : ppe_finish_mode<PPE_MODE_SLOPE>(v, pu);
+        }
+        packed |= ((uint32_t)y & 0xFFu) << (8 * i);
+    }
+    if (store) {
+        uint8_t* const dst = t.out.data + (int64_t)n * t.out.sn + (int64_t)oy * t.out.sh + (int64_t)ox * t.out.sw + (int64_t)(oc + 4 * part) * t.out.sc;
+        if (t.out.sc == 1) {
+            *reinterpret_cast<uint32_t*>(dst) = packed;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dst[i * t.out.sc] = (uint8_t)(packed >> (8 * i));
+        }
+    }
+}
+
+// hipErrorNotSupported: more items than the kernel counts.
+hipError_t launch_avgpool_split(const TaskDev& t, const Box& box, hipStream_t s) {
+    SplitArgs a;
+    a.t = t;
+    a.box = box;
+    const int32_t cgroups = box.bc >> 4;
+    const int64_t npix = (int64_t)t.out.n * box.bh * box.bw;
+    if (npix == 0 || cgroups == 0) return hipSuccess;
+    a.glog = cgroups >= 8 ? 3 : cgroups >= 4 ? 2 : cgroups >= 2 ? 1 : 0;
+    a.nslabs = (uint32_t)((cgroups + (1 << a.glog) - 1) >> a.glog);
+    if (npix * a.nslabs > 0x7ffffff0LL) return hipErrorNotSupported;
+    a.nitems = (uint32_t)(npix * a.nslabs);
+    a.ntaps = t.ky * t.kx;
+    a.div_slabs = make_fastdiv(a.nslabs);
+    a.div_bw = make_fastdiv((uint32_t)box.bw);
+    a.div_bh = make_fastdiv((uint32_t)box.bh);
+    a.div_kx = make_fastdiv((uint32_t)t.kx);
+    a.a_xor = t.in.is_signed ? 0x80808080u : 0u;
+    a.zpu = t.in.zp + (t.in.is_signed ? 128 : 0);
+    a.fill = (uint32_t)a.zpu * 0x01010101u;
+    return emit(avgpool_split_kernel, dim3((a.nitems + NT / 64 - 1) / (NT / 64)), dim3(NT), 0, s, a);
+}
+
 template <int MODE, int KK, bool I32>
 hipError_t launch_window_i32(const WinArgs& a, int64_t blocks, int nslabs, size_t lds, hipStream_t s) {
     static LdsGrant grant;  // large depthwise kernels: opt in to more than the default dynamic LDS
@@ -423,6 +572,10 @@ hipError_t launch_window(const TaskDev& t, const Box& box, hipStream_t s) {
     if (t.ky == 3 && t.kx == 3) return launch_window_kk<MODE, 3>(t, box, s);
     if (t.ky == 2 && t.kx == 2) return launch_window_kk<MODE, 2>(t, box, s);
     if (t.ky == 5 && t.kx == 5) return launch_window_kk<MODE, 5>(t, box, s);
+    if (MODE == MODE_AVG && t.ky * t.kx > 9) {  // (fewer taps than lanes to give them to are not worth the exchanges)
+        const hipError_t e = launch_avgpool_split(t, box, s);
+        if (e != hipErrorNotSupported) return e;
+    }
     return launch_window_kk<MODE, 0>(t, box, s);
 }
 
