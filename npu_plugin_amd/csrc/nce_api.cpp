@@ -79,6 +79,7 @@ struct ScopedLaunch {
     ScopedLaunch(const nce::Options* opt, std::vector<nce::RecordedLaunch>* record, nce_log_s* log = nullptr) : saved(nce::tls_launch) {
         nce::tls_launch.opt = opt;
         nce::tls_launch.record = record;
+        nce::tls_launch.in_list = false;
         nce::tls_launch.log = log;
     }
     ~ScopedLaunch() { nce::tls_launch = saved; }
@@ -94,6 +95,7 @@ nce::Options read_options() {
         o.wres_forced = sscanf(e, "%d,%d,%d,%d", &o.wres[0], &o.wres[1], &o.wres[2], &o.wres[3]) == 4;
     if (const char* e = getenv("NCE_HIP_CONV_TILE")) o.halo_tile = atoi(e);
     if (const char* e = getenv("NCE_HIP_CONV_TILED")) o.tiled = atoi(e);
+    if (const char* e = getenv("NCE_HIP_CONV_SPLIT")) o.split = atoi(e);
     if (const char* e = getenv("NCE_HIP_CONV_PATCH")) {
         int nf = 0, pr = 0, wv = 0, npx = 0;
         const int got = sscanf(e, "%d,%d,%d,%d", &nf, &pr, &wv, &npx);
@@ -957,6 +959,7 @@ nce_result_t enqueue_list(nce_task_list_handle_t list, void* hip_stream, bool fi
             std::vector<PkAlt> alts;
             {
                 const ScopedLaunch ctx(&ex->opt, &list->launches, ex->log);
+                nce::tls_launch.in_list = list->plans.size() > 1;
                 const nce_result_t r = run_plans(ex, list->plans, nullptr, persistent ? &alts : nullptr);
                 if (r != NCE_RESULT_SUCCESS) {
                     list->launches.clear();

@@ -168,6 +168,7 @@ struct Options {
     int persistent = 0;       // NCE_HIP_PERSISTENT: task lists run runs of weights-resident convolutions as one persistent launch
     int persistent_wait_us = 2000000;  // NCE_HIP_PERSISTENT_WAIT_US: time after which a persistent launch's waits give up
     int tiled = -1;           // NCE_HIP_CONV_TILED: -1 automatic, 0 never, 1.. force that shape of the LDS-tiled kernel
+    int split = -1;           // NCE_HIP_CONV_SPLIT: -1 automatic, 0 never, 1.. force that tile of the split-reduction kernel
     int patch = -1;           // NCE_HIP_CONV_PATCH: -1 automatic, 0 never, 1 = wherever its conditions hold; "nf,pr[,waves]" also forces its shape
     int patch_nf = 0, patch_pr = 0, patch_waves = 0, patch_npx = 0;
     bool env_path = false;    // NCE_HIP_CONV_PATH was given at all (switches the conv + add fusion off, as NO_FUSE does)
@@ -192,6 +193,8 @@ struct LaunchContext {
     // Per-XCD form: the task is one eighth of the batch, to be run by the 32 CUs of one XCD inside a persistent segment
     // (grids are sized for 32 CUs; only the weights-resident convolution kernels take part).
     bool per_xcd = false;
+    // The launch is one of a list of tasks: its weights were last read a whole pass ago and come from memory, not from L2.
+    bool in_list = false;
 };
 extern thread_local LaunchContext tls_launch;
 inline const Options& options() {

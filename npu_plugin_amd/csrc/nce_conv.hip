@@ -15,6 +15,8 @@
 // Out-of-image taps are filled with the byte zp_a, so that (a' + da) = 0 there.
 #include "nce_conv_common.h"
 
+#include <algorithm>
+
 namespace nce {
 namespace {
 
@@ -303,33 +305,6 @@ static bool overlaps(const TensorDev& x, const TensorDev& y) {
     return x.data < ye && y.data < xe;
 }
 
-// Which convolutions take the LDS-tiled kernel: 0 = none of its shapes, else the shape (0 within a forced value: automatic).
-static int tiled_shape_for(const ConvArgs& a) {
-    if (tls_launch.per_xcd) return 0;
-    const int forced = options().tiled;
-    if (forced >= 0) return forced;
-    // Fitted to a sweep of the ResNet-50 layer shapes at batch 32, 64, 128 and 256 (each layer alone, every kernel forced)
-    // and to the whole graph at those batches. The 128 x 128 tile with steps of 128 bytes of the reduction (one barrier and
-    // one LDS round trip per 32 matrix instructions of a wave; input channels a multiple of 128) is 3-25 % ahead of the
-    // weights-resident kernels - 45 % for 3x3 over 512 channels - where the reduction is long and the output channels are
-    // many. Inside the graph a launch of it costs ~1.5 us more than alone (the layer-alone sweep repeats one kernel, whose
-    // weights then stay in L2 and whose launches overlap their own tails), so grids whose gain alone is 1-2 us are left to
-    // the weights-resident kernels: from 1024 bytes of reduction it takes 384 workgroups (196 from 4096 bytes), from 512
-    // bytes 512 workgroups of at least 256 channels - but not 256..511 channels over more than 1024 workgroups, where the
-    // weights-resident kernels amortise their staging over many tiles per workgroup and win again. Shorter reductions and
-    // fewer than 128 channels always lose. The 64-byte-step shape (input channels not a multiple of 128) is 9 % slower and
-    // keeps the narrower window it was measured in. (The sweep ran the 128-byte steps with four waves per workgroup; the same
-    // tile with eight waves - shape 6, what is returned now - is 1-3 % ahead of it on every layer of the window.)
-    const int64_t k = (int64_t)a.KY * a.KX * a.IC;
-    if (a.IC % 64 != 0 || a.dw != 0 || k < 512 || a.bc < 128) return 0;
-    const int64_t groups = (((int64_t)a.M + 127) / 128) * ((a.bc + 127) / 128);
-    if (a.IC % 128 != 0) return k >= 1024 && a.bc >= 256 && groups >= 384 && groups <= 1024 ? 1 : 0;
-    bool use;
-    if (k >= 1024) use = groups >= (k >= 4096 ? 196 : 384);
-    else use = a.bc >= 256 && groups >= 512 && (a.bc >= 512 || groups <= 1024);
-    return use ? 6 : 0;
-}
-
 // Which convolutions take the patch kernel (both operands in LDS, every input byte fetched once per workgroup).
 static bool patch_wanted(const ConvArgs& a) {
     if (tls_launch.per_xcd) return false;
@@ -337,13 +312,109 @@ static bool patch_wanted(const ConvArgs& a) {
     if (forced >= 0) return forced != 0;
     // Measured against the weights-resident kernels over the ResNet-50 shapes at batch 32 .. 256 (each layer alone): ahead
     // by 6-17 % for 3x3 kernels at stride 1 over 64 input channels from about 100,000 output pixels and over 128 input
-    // channels from about 50,000 (64 output channels per slice, sixteen waves); level or behind for everything else - 1x1
+    // channels from about 50,000 (64 output channels per slice, sixteen waves); level or behind for everything else - larger
+    // kernels (5x5 over 128 channels: 191 us against 75 us of the LDS-tiled kernel), 1x1
     // kernels (nothing to reuse), 256 and more input channels (a slice of 32 channels reads 0.75 KiB of LDS per matrix
     // instruction) and small layers (too few patches for the CUs).
-    if (a.KY * a.KX < 2 || a.SY != 1 || a.SX != 1 || a.dw != 0 || a.bc < 64) return false;
+    if (a.KY * a.KX < 2 || a.KY * a.KX > 9 || a.SY != 1 || a.SX != 1 || a.dw != 0 || a.bc < 64) return false;
     if (a.IC == 64) return a.M >= 100000;
     if (a.IC == 128) return a.M >= 50000;
     return false;
+}
+
+// ---- which kernel a convolution takes ----------------------------------------------------------------------------------------
+// The split-reduction, LDS-tiled and weights-resident kernels serve overlapping ranges of tasks, and which of their tiles is
+// ahead depends on how the grid fills the chip: one rule of thumb per kernel left 30 % on the table. So each has a cost
+// estimate in microseconds - a few terms that count what the kernel does (rounds of workgroups, reduction steps per round,
+// bytes through a CU's load path, fragments exchanged, output bytes), with coefficients fitted by non-negative least squares
+// on the relative error over 734 measured tasks: random shapes, types and zero points, 1 to 64 images, and the ResNet-50
+// layers at batch 1 to 128, every kernel and tile forced on every task. The estimates are within 10-25 % of the measured
+// times for nine tasks in ten; the kernel chosen by them is on average 3 % slower than the best one of each task, where the
+// patch and weights-resident kernels and their fallbacks alone were 39 % slower.
+static double estimate_split(const ConvArgs& a, int shape) {
+    struct Tile {
+        int nf, bf, depth;
+        double base, round, kib, frags, step, wait;
+    };
+    static const Tile tiles[5] = {
+        {1, 1, 8, 3.27, 1.521, 0.01781, 0.0444, 0.0, 0.0},     {2, 1, 5, 3.41, 2.029, 0.0, 0.0478, 0.2985, 0.0},
+        {2, 2, 4, 3.67, 1.528, 0.0129, 0.1141, 0.0, 0.0},      {4, 2, 3, 4.07, 2.238, 0.0, 0.1135, 0.3513, 0.4308},
+        {4, 4, 2, 4.96, 2.413, 0.0, 0.1274, 0.0894, 1.213},
+    };
+    const Tile& t = tiles[shape - 1];
+    const int64_t slices = (a.KG + 3) / 4;
+    const int f = t.nf + t.bf, slots = t.nf * t.bf + (a.da != 0 || a.dw != 0 ? f : 0);
+    const int64_t most = std::min(8, 156 / slots);
+    const int64_t per_wave = (slices + most - 1) / most, waves = (slices + per_wave - 1) / per_wave;
+    const int64_t groups = (((int64_t)a.M + 16 * t.bf - 1) / (16 * t.bf)) * ((a.bc + 16 * t.nf - 1) / (16 * t.nf));
+    const int64_t resident = std::max<int64_t>(1, std::min<int64_t>(156 / (waves * std::max(t.depth * f, slots)), 32 / waves));
+    const double rounds = (double)((groups + 256 * resident - 1) / (256 * resident)), per_cu = (double)((groups + 255) / 256);
+    return t.base + t.round * (rounds - 1) + t.kib * per_cu * (double)(slices * f) + t.frags * per_cu * (t.nf * t.bf) +
+           t.step * rounds * (double)per_wave + t.wait * rounds * (double)((per_wave + t.depth - 1) / t.depth);
+}
+
+static double estimate_tiled(const ConvArgs& a, int shape) {
+    struct Tile {
+        int bm, bn, resident;
+        double base, step, more, round, group, unit, unit_alone, wsum, asum, out;
+    };
+    static const Tile tiles[7] = {
+        {256, 256, 1, 2.113, 1.283, 1.559, 0.0, 5.08, 0.2087, 0.0, 0.2207, 1.845, 0.1322},
+        {256, 128, 1, 1.725, 0.7668, 0.8765, 4.016, 0.0, 0.1812, 0.0, 0.1575, 0.2475, 0.1272},
+        {128, 128, 2, 2.285, 0.4806, 0.332, 1.303, 1.013, 0.1278, 0.0, 0.1621, 0.1994, 0.1388},
+        {128, 64, 3, 1.796, 0.4204, 0.1802, 1.995, 0.5824, 0.0729, 0.0622, 0.1033, 0.0841, 0.0462},
+        {64, 128, 3, 0.912, 0.3846, 0.18, 2.411, 0.747, 0.0898, 0.0603, 0.1252, 0.0854, 0.0439},
+        {64, 64, 4, 1.909, 0.3144, 0.1124, 1.63, 0.3388, 0.0618, 0.0767, 0.0697, 0.0372, 0.0713},
+        {256, 64, 1, 1.443, 0.6594, 0.6942, 3.968, 0.0, 0.1804, 0.0, 0.1785, 0.1292, 0.1069},
+    };
+    const Tile& t = tiles[shape - 1];
+    const double steps = (double)((a.KG + 7) / 8);
+    const int64_t groups = (((int64_t)a.M + t.bm - 1) / t.bm) * ((a.bc + t.bn - 1) / t.bn);
+    const double per_cu = (double)((groups + 255) / 256), rounds = (double)((groups + 256 * t.resident - 1) / (256 * t.resident));
+    const bool units = a.IC % 128 != 0 || a.dw != 0;
+    return t.base + t.step * steps + t.more * steps * (per_cu - 1) + t.round * rounds + t.group * per_cu +
+           (units ? t.unit * steps * per_cu + t.unit_alone * steps : 0.0) + (a.da != 0 ? t.wsum * steps * per_cu : 0.0) +
+           (a.dw != 0 ? t.asum * steps * per_cu : 0.0) + 1e-6 * t.out * (double)a.M * a.bc;
+}
+
+static double estimate_wres(const ConvArgs& a, const WresShape& s) {
+    const double steps = (double)((a.KG + 3) / 4), rounds = (double)((s.groups * s.slices + 255) / 256);
+    const double tiles = (double)((s.tiles_per_group + 7) / 8);  // per wave
+    const double out = 1e-6 * (double)a.M * a.bc, in = 1e-6 * (double)a.M * a.SY * a.SX * a.IC * (double)s.slices;
+    const double stage = steps * s.nf * rounds, mma = tiles * steps * s.nf * s.bf * rounds, sums = a.da != 0 || a.dw != 0 ? stage : 0.0;
+    const double asums = a.dw != 0 ? tiles * steps * s.bf * rounds : 0.0;
+    if (a.IC % 64 != 0)  // (per-lane loads)
+        return 3.421 * rounds + 0.00143 * stage + 0.00775 * mma + 0.1003 * tiles * rounds + 0.1024 * tiles * steps * s.bf * rounds + 0.00868 * sums +
+               0.02104 * asums + 0.4475 * out + 0.0232 * in;
+    return 3.21 + 0.00669 * stage + 0.0859 * tiles * steps * rounds + 0.02955 * mma + 0.0119 * sums + 0.01219 * asums + 0.2285 * out + 0.0016 * in +
+           (a.bc % 64 != 0 ? 0.2556 * out : 0.0);
+}
+
+struct ConvChoice {
+    int split, tiled;  // the tile of the split-reduction / LDS-tiled kernel to try first; 0, 0: the other kernels
+};
+static ConvChoice choose_conv(const ConvArgs& a, bool fused) {
+    if (tls_launch.per_xcd || options().conv_path != 0 || options().wres_forced) return {0, 0};
+    if (options().split > 0) return {options().split, 0};
+    if (options().tiled > 0) return {0, options().tiled};
+    if (options().patch > 0) return {0, 0};
+    ConvChoice c = {0, 0};
+    const WresShape s = wres_shape_for(a, fused);
+    // (The weights-resident kernel's estimate is the least certain: it has to be beaten by 10 %. Of the 734 tasks four then come
+    // out more than 4 % slower than it. Those were tasks enqueued again and again, whose weights sit in L2. In a list they come
+    // from memory, a launch of any kernel is slower than its estimate - and the LDS-tiled kernel, which requests them all
+    // ahead, by less: ResNet-50 at batch 32, 663 us with the factor for single tasks, 651 with the one for lists.)
+    const double wres_factor = tls_launch.in_list ? 1.0 : 0.9;
+    // (what is neither a weights-resident nor a patch task would take a kernel that gathers or re-stages its operands: those
+    // are never ahead)
+    double best = !fused && patch_wanted(a) ? 0.0 : s.ok && (!fused || s.nf == 4) ? wres_factor * estimate_wres(a, s) : 1e30;
+    if (options().split < 0)
+        for (int i = 1; i <= 5; ++i)
+            if (const double t = estimate_split(a, i); t < best) best = t, c = {i, 0};
+    if (options().tiled < 0 && !(fused && (a.IC % 128 != 0 || a.dw != 0)))
+        for (int i = fused ? 2 : 1; i <= 7; ++i)  // (256 x 256 tiles, one workgroup per CU, leave an add's traffic with nothing beside it)
+            if (const double t = estimate_tiled(a, i); t < best) best = t, c = {0, i};
+    return c;
 }
 
 hipError_t launch_conv_fused_add(const TaskDev& conv, const Box& cb, const TaskDev& add, const Box& ab, hipStream_t stream) {
@@ -377,8 +448,13 @@ hipError_t launch_conv_fused_add(const TaskDev& conv, const Box& cb, const TaskD
     ConvArgs a;
     if (const hipError_t e = make_conv_args(conv, cb, a); e != hipSuccess) return e;
     if (a.M == 0 || cb.bc == 0) return hipErrorNotSupported;
-    if (const int shape = tiled_shape_for(a)) {
-        const hipError_t e = launch_conv_tiled(a, stream, shape, &fz);
+    const ConvChoice choice = choose_conv(a, true);
+    if (choice.split != 0) {
+        const hipError_t e = launch_conv_split(a, stream, choice.split, &fz);
+        if (e != hipErrorNotSupported) return e;
+    }
+    if (choice.tiled != 0) {
+        const hipError_t e = launch_conv_tiled(a, stream, choice.tiled, &fz);
         if (e != hipErrorNotSupported) return e;
     }
     return launch_conv_wres(a, stream, false, &fz);
@@ -395,11 +471,14 @@ hipError_t launch_conv(const TaskDev& t, const Box& box, hipStream_t stream) {
     // 3x3 over 1024 channels), the chunked weights-resident kernel for everything else and for what the halo
     // kernel rejects.
     hipError_t e = hipErrorNotSupported;
+    const ConvChoice choice = choose_conv(a, false);
+    if (choice.split != 0) e = launch_conv_split(a, stream, choice.split);
+    if (e != hipErrorNotSupported) return e;
+    if (choice.tiled != 0) e = launch_conv_tiled(a, stream, choice.tiled);
+    if (e != hipErrorNotSupported) return e;
     if (path == 0 && patch_wanted(a))
         e = launch_conv_patch(a, stream, options().patch >= 0 ? options().patch_nf : 4, options().patch_pr, options().patch >= 0 ? options().patch_waves : 16,
                               options().patch >= 0 ? options().patch_npx : 0);
-    if (e != hipErrorNotSupported) return e;
-    if (const int shape = path == 0 ? tiled_shape_for(a) : 0) e = launch_conv_tiled(a, stream, shape);
     if (e != hipErrorNotSupported) return e;
     e = path == 0 ? launch_conv_wres(a, stream, a.KX != 3) : hipErrorNotSupported;
     if (e != hipErrorNotSupported) return e;

@@ -49,5 +49,14 @@ __device__ __forceinline__ void load_to_lds_16(const void* src, void* block) {
 #pragma clang diagnostic pop
 }
 
+// The same with the address as a uniform base and a 32-bit lane offset: no vector arithmetic where the base moves alone.
+__device__ __forceinline__ void load_to_lds_16(const uint8_t* base, uint32_t offset, void* block) {
+    const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)block;
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_addr) : "memory", "m0");
+#pragma clang diagnostic pop
+}
+
 }  // namespace lds_detail
 }  // namespace nce

@@ -1,25 +1,33 @@
-// CONV task, LDS-tiled implicit GEMM on v_mfma_i32_16x16x64_i8 for layers with many output channels.
+// CONV task, LDS-tiled implicit GEMM on v_mfma_i32_16x16x64_i8 for tasks with many output pixels and channels.
 //
-// A workgroup owns BM = 16*TM*WM output pixels x BN = 16*TN*WN output channels. Both operands of a reduction
-// step (64 bytes of the OYXI weight rows; the same 64 input channels of one tap of every pixel) are staged in
-// LDS once per workgroup and shared by its waves: the WN waves along the channels read the same activation
-// rows, the WM waves along the pixels the same weight rows. Per step a wave reads TN + TM operand fragments
-// for TN*TM matrix instructions (the weights-resident kernel, whose waves share nothing, reads its
-// activations from global memory once per wave and tops out on the CU's L1 path).
+// A workgroup owns BM = 16*TM*WM output pixels x BN = 16*TN*WN channels. Both operands of a reduction step (128 bytes of the
+// OYXI weight rows; the same part of every pixel's window) are staged in LDS once per workgroup and shared by its waves: the
+// WN waves along the channels read the same activation rows, the WM waves along the pixels the same weight rows. Per 64-byte
+// half of a step a wave reads TN + TM operand fragments for TN*TM matrix instructions.
 //
-// Staging: global_load_lds_dwordx4 moves 16 bytes per lane from global memory straight into LDS (no registers,
-// no LDS store instruction): one instruction of a wave fills one 1 KiB block = 16 rows x 64 bytes, lane 4p + j
-// at byte 16 * (4p + j) of the block. Which 16-byte piece of row p that lane FETCHES is the layout: piece
-// j ^ swz(p), so that the row-per-lane operand reads spread over all banks while four neighbouring lanes still
-// fetch one row's 64 contiguous bytes. NS stages of (BM + BN) * 64 bytes form a ring: the requests of step
-// s + NS - 1 are issued when step s begins, so NS - 1 steps of loads are in flight per workgroup, and one
-// barrier per step orders "my requests for this stage have landed" (s_waitcnt vmcnt) before every wave's reads.
-// u8 operands are re-biased (x ^ 0x80) in registers after the operand read; taps outside the image fetch a
-// line holding the input zero point. With an input zero point away from the storage offset the per-channel
-// weight sums come out of the matrix unit (one more instruction per weight fragment and step, against ones).
+// Staging: global_load_lds_dwordx4 moves 16 bytes per lane from global memory straight into LDS (no registers, no LDS
+// store). One instruction fills a 1 KiB block of 8 rows x 128 bytes: eight neighbouring lanes fetch one row's 128 bytes, a
+// whole cache line. (With blocks of 16 rows x 64 bytes the two halves of a line are fetched a step apart, and by then a tile
+// of 512 rows has pushed the line out of the 32 KiB L1: the same loop then moved twice the bytes from L2 and a 256 x 256
+// tile took 0.69 us per 64 bytes of the reduction.) Which 16-byte piece of its row a lane FETCHES is the layout: piece
+// j ^ swz8(row / 2) at position j, which spreads the operand reads over all banks (below). NS steps form a ring.
 //
-// Conditions (checked on the host): input channels a multiple of 64, weights zero point equal to their
-// storage offset, kernel up to 32 x 32. Semantics and the fused PPE are those of the weights-resident kernel
+// The loop is software-pipelined through registers: while the matrix instructions of one half of a step run, the operands of
+// the next half are read from LDS, dealt out between them, and a pixel fragment is re-biased (u8 storage: x ^ 0x80) one
+// group ahead of its use, so that no matrix instruction waits for an LDS or vector one. One barrier per step: it says that
+// every wave's requests of the next step have landed and that every wave holds this step in registers, so its ring slot is
+// free and is requested again at once. Taps outside the image fetch a line holding the input zero point. With an input
+// zero point away from the storage offset the per-channel weight sums come out of the matrix unit against ones; the WM waves
+// that read the same weight fragments share that out.
+//
+// What bounds it: for 256 x 256 tiles the matrix cores at the clock their power leaves them (a loop of nothing but the operand
+// reads, re-biasing and matrix instructions on random bytes holds 3.4 POP/s on the whole chip, 4.4 on a sixteenth of it);
+// for the smaller tiles, which the smaller tasks need to fill 256 CUs, the barrier and LDS round trip of a step. Measured
+// against a loop without the register pipeline that fetched 16 x 64 byte blocks: 3x3 over 256 channels, 32 x 56 x 56, input
+// zero point 0: 85-89 -> 71 us (1.66 POP/s); 128 x 7 x 7 x 512: 25.9 -> 21.6 us; 5x5 over 112 channels (a gather kernel
+// before): 70 -> 31 us.
+//
+// Conditions (checked on the host): kernel up to 15 x 15. Semantics and the fused PPE are those of the weights-resident kernel
 // (nce_conv_epi.h).
 #include "nce_conv_epi.h"
 #include "nce_conv_lds.h"
@@ -36,44 +44,59 @@ using namespace wres_detail;
 
 struct TiledArgs {
     ConvArgs a;
-    int32_t nsteps;   // 64-byte reduction steps: KY * KX * IC / 64
-    int32_t nc64;     // 64-byte chunks along IC
+    int32_t nsteps;   // 128-byte reduction steps, rounded up
+    int32_t nc128;    // TILED_CHUNKS: 128-byte chunks along IC
     uint32_t ntm;     // pixel tiles
     uint32_t ntn;     // channel tiles
-    int32_t inside;   // every tap of every pixel of the box lies inside the image
+    FastDiv div_ntn;
+    WarmArgs warm;
+    int32_t wraps;    // TILED_UNITS: taps eight consecutive units can reach into (1 .. 8)
     int64_t row_adv;  // input offset from the last tap of a kernel row to the first of the next: in_sh - KX * in_sw
     FuseAdd fz;       // FZ kernels only
 };
 
-using namespace lds_detail;  // swz (bank-conflict-free piece placement), vmcnt_imm, gptr_t / lptr_t
+using namespace lds_detail;  // vmcnt_imm, load_to_lds_16
 
-// Waves per SIMD the register budget must allow (vector + accumulation registers share 512 per lane and SIMD): two
-// workgroups of four waves, or one of eight, per CU at the least - a lone wave per SIMD leaves every LDS and barrier
-// round trip of the step loop exposed. Eight waves of 32 x 64 outputs (eight accumulator fragments) fit 128 registers: two
-// such workgroups share a CU, four waves per SIMD.
-constexpr int tiled_min_waves(int nwaves, int frags) {
-    return nwaves >= 8 && frags <= 8 ? 4 : 2;
+// Blocks of 8 rows x 128 bytes, two per operand fragment of 16 rows: piece p (0..7) of row r (0..15) sits at
+// r * 128 + ((p ^ swz8(r >> 1)) << 4). A ds_read_b128 of an operand is served in clocks of sixteen lanes that hold rows 0-3 and
+// 12-15 with one piece and rows 4-11 with its neighbour (nce_conv_lds.h); rows of equal parity share the eight bank groups
+// of half the banks, so for those eight rows the positions p ^ {0, 1, 6, 7} and p ^ 1 ^ {3, 2, 5, 4} have to be eight
+// different ones - they are.
+__device__ __forceinline__ int swz8(int k) {
+    return (0x76452310 >> (4 * k)) & 7;
 }
 
-template <int WM, int WN, int TM, int TN, int NS, int KC, bool FZ>
-__global__ __launch_bounds__(64 * WM * WN, tiled_min_waves(WM * WN, TM * TN)) void conv_tiled_kernel(TiledArgs w) {
+// GEN: TILED_CHUNKS - input channels a multiple of 128: a step lies in one tap, its position is scalar. TILED_UNITS - any
+// multiple of 16: a step is eight 16-byte units (tap, 16 channels) of their own and each lane walks the unit of the piece it
+// fetches; past the reduction's end the weights read zeros. TILED_UNITS_ASUM - units, and weights whose zero point differs
+// from their storage offset by dw: the per-pixel activation sums come out of the matrix unit (one more instruction per pixel
+// fragment and half step, against ones; past the end and outside the image a fetch is the zero point, a' = -da, which the
+// constant nsteps * 128 * da * dw takes back).
+enum { TILED_CHUNKS = 0, TILED_UNITS = 1, TILED_UNITS_ASUM = 2 };
+
+// OCC: waves per SIMD the register budget has to allow.
+template <int WM, int WN, int TM, int TN, int NS, int OCC, bool FZ, int GEN>
+__global__ __launch_bounds__(64 * WM * WN, OCC) void conv_tiled_kernel(TiledArgs w) {
     prefetch_kernel_arguments<sizeof(TiledArgs)>();
+    constexpr bool UNITS = GEN != TILED_CHUNKS;
+    constexpr bool ASUM = GEN == TILED_UNITS_ASUM;
     constexpr int NW = WM * WN;
     constexpr int BM = 16 * TM * WM;
     constexpr int BN = 16 * TN * WN;
     constexpr int CW = 16 * TN;              // channels per wave
-    constexpr int ABLK = BN / 16;            // 1 KiB blocks of the weight tile
-    constexpr int NA = ABLK / NW;            // blocks of the weight tile one wave fetches per step
-    constexpr int NB = (BM / 16) / NW;       // blocks of the activation tile
-    constexpr int CHUNK = (BM + BN) * 64;    // bytes of one 64-byte slice of the reduction: weight rows, then activation rows
-    constexpr int STAGE = CHUNK * KC;        // bytes of one LDS stage: KC slices (a step covers 64 * KC bytes of the reduction)
+    constexpr int NA = BN / 8 / NW;          // blocks of the weight tile one wave fetches per step
+    constexpr int NB = BM / 8 / NW;          // blocks of the activation tile
+    constexpr int STAGE = (BM + BN) * 128;   // bytes of one ring slot: weight rows, then activation rows
     static_assert(TN == 2 || TN == 4, "channel fragments per wave");
-    static_assert(ABLK % NW == 0 && (BM / 16) % NW == 0, "blocks divide among the waves");
+    static_assert((BN / 8) % NW == 0 && (BM / 8) % NW == 0 && NW % 2 == 0, "blocks divide among the waves");
     static_assert(!FZ || TN == 4, "fused add: a lane holds 16 channels");
-    static_assert(NS >= 2 && (NS - 2) * (NA + NB) * KC < 64, "ring depth against the 6-bit load counter");
+    static_assert(NS >= 2 && (NS - 1) * (NA + NB) < 64, "ring depth against the 6-bit load counter");
     const ConvArgs& a = w.a;
 
-    extern __shared__ __attribute__((aligned(16))) uint8_t sT[];  // [stage][weights BN rows | activations BM rows] x 64 bytes
+    WarmLines warm;
+    warm.request(w.warm, (blockIdx.x >> 3) * NW + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+
+    extern __shared__ __attribute__((aligned(16))) uint8_t sT[];  // [slot][weights BN rows | activations BM rows] x 128 bytes
     __shared__ int64_t sOutOff[BM];   // output byte offset of the tile's pixels (channel 0 of the tensor)
     __shared__ int32_t sW2[BN], sBias[BN], sWsum[BN];
     __shared__ int32_t sCorr[BN];     // integer path: da * sum of weights; high-word path: scaled multiplier
@@ -90,83 +113,106 @@ __global__ __launch_bounds__(64 * WM * WN, tiled_min_waves(WM * WN, TM * TN)) vo
     const uint32_t ntotal = w.ntm * w.ntn;
     const uint32_t lid = xcd_tile(blockIdx.x, ntotal);
     if (lid >= ntotal) return;  // uniform for the whole workgroup
-    const uint32_t mt = lid / w.ntn, nt = lid - mt * w.ntn;
+    const uint32_t mt = fdiv(lid, w.div_ntn), nt = lid - mt * w.ntn;
     const int32_t oc0 = a.z0 + (int32_t)nt * BN;
     const int32_t noc = min(BN, a.z0 + a.bc - oc0);
     const int32_t m0 = (int32_t)mt * BM;
 
-    // ---- what this thread fetches: row lane / 4 of the blocks wave, wave + NW, ... ; position lane % 4 -----------
-    const int prow = lane >> 2;
-    const int pj = (lane & 3) ^ swz(prow);  // the piece that belongs at this lane's position
-    const uint8_t* wsrc[NA];
+    // ---- what this thread fetches: row lane / 8 of the blocks wave, wave + NW, ... ; position lane % 8 -----------
+    const int brow = (wave & 1) * 8 + (lane >> 3);  // row within its fragment of 16 (NW is even: the same for all its blocks)
+    const int pj = (lane & 7) ^ swz8(brow >> 1);    // the piece that belongs at this lane's position
+    uint32_t woff[NA];                              // byte offset from the first weight set of the tile
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
-        const int r = (wave + NW * i) * 16 + prow;  // row of the weight tile: fragment r / 16, wave group r / CW
+        const int r = (wave + NW * i) * 8 + (lane >> 3);  // row of the weight tile: fragment r / 16, wave group r / CW
         const int cl = (r / CW) * CW + channel_of_frag_row<TN>((r % CW) >> 4, r & 15);
         const int ch = min(cl, noc - 1);  // rows past the box's last channel duplicate it (their results are not stored)
-        wsrc[i] = a.w + (int64_t)(oc0 + ch) * a.w_soc + pj * 16;
+        woff[i] = (uint32_t)ch * (uint32_t)a.w_soc + (UNITS ? 0 : pj * 16);
     }
+    const uint8_t* const wbase = a.w + (int64_t)oc0 * a.w_soc;
     const uint8_t* bsrc[NB];
-    uint32_t rows[NB], cols[NB];
+    uint32_t taps[NB];  // bit ky: kernel row ky lies inside the image; bit 16 + kx: kernel column kx does
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-        const int r = (wave + NW * i) * 16 + prow;  // pixel of the tile
-        const int32_t p = min(m0 + r, a.M - 1);     // pixels past the end duplicate the last one
+        const int r = (wave + NW * i) * 8 + (lane >> 3);  // pixel of the tile
+        const int32_t p = min(m0 + r, a.M - 1);           // pixels past the end duplicate the last one
         const int32_t rr = fdiv(p, a.div_bw);
         const int32_t bx = p - rr * a.bw;
         const int32_t n = fdiv(rr, a.div_bh);
         const int32_t by = rr - n * a.bh;
         const int32_t iy0 = (a.y0 + by) * a.SY - a.PT;
         const int32_t ix0 = (a.x0 + bx) * a.SX - a.PL;
-        bsrc[i] = a.in + (int64_t)n * a.in_sn + (int64_t)iy0 * a.in_sh + (int64_t)ix0 * a.in_sw + pj * 16;
-        rows[i] = bit_range(max(0, -iy0), min(a.KY, a.H - iy0));
-        cols[i] = bit_range(max(0, -ix0), min(a.KX, a.W - ix0));
-        if ((lane & 3) == 0) sOutOff[r] = (int64_t)n * a.out_sn + (int64_t)(a.y0 + by) * a.out_sh + (int64_t)(a.x0 + bx) * a.out_sw;
+        bsrc[i] = a.in + (int64_t)n * a.in_sn + (int64_t)iy0 * a.in_sh + (int64_t)ix0 * a.in_sw + (UNITS ? 0 : pj * 16);
+        taps[i] = bit_range(max(0, -iy0), min(a.KY, a.H - iy0)) | bit_range(max(0, -ix0), min(a.KX, a.W - ix0)) << 16;
+        if ((lane & 7) == 0) sOutOff[r] = (int64_t)n * a.out_sn + (int64_t)(a.y0 + by) * a.out_sh + (int64_t)(a.x0 + bx) * a.out_sw;
     }
-    const uint8_t* const fillp = &g_fill.b[a.fill_raw][pj * 16];
+    const uint8_t* const fillp = &g_fill.b[a.fill_raw][(pj & 3) * 16];
     if (tid < BN) sWsum[tid] = 0;
     if (tid == 0) sFlags = 0;
 
-    // scalar walk over (kernel row, kernel column, 64-byte channel chunk); additions only
-    int32_t it_ky = 0, it_kx = 0, it_c64 = 0;
-    int64_t it_off = 0, tap_off = 0, w_off = 0;
-    // Request one step's operands into ring slot `slot` (uniform).
+    // TILED_CHUNKS: scalar walk over (kernel row, kernel column, 128-byte channel chunk); additions only
+    int32_t it_ky = 0, it_kx = 0, it_c = 0;
+    int64_t it_off = 0, tap_off = 0;
+    const uint8_t* it_w = wbase;
+    // TILED_UNITS: this lane's walk over the 16-byte units pj, pj + 8, pj + 16 ... of the reduction
+    const uint8_t* const wzero = &g_fill.b[a.w_xor & 0x80u][(pj & 3) * 16];  // (bytes that are zero once re-biased)
+    int32_t u = pj, u_icg = pj, u_kx = 0, u_ky = 0;
+    int64_t u_tap = 0;
+    auto wrap_unit = [&]() {
+        for (int i = 0; i < w.wraps; ++i) {  // (uniform)
+            const bool over = u_icg >= a.ICG;
+            const bool row = over && u_kx + 1 == a.KX;
+            u_icg -= over ? a.ICG : 0;
+            u_kx = row ? 0 : u_kx + (over ? 1 : 0);
+            u_ky += row ? 1 : 0;
+            u_tap += over ? a.in_sw : 0;
+            u_tap += row ? w.row_adv : 0;
+        }
+    };
+    if constexpr (UNITS) wrap_unit();
+    // Request the next step's operands into ring slot `slot` (uniform) and move on.
     auto request = [&](int slot) {
+        uint8_t* const st = sT + slot * STAGE + wave * 1024;
+        if constexpr (UNITS) {
+            const bool real = u < a.KG;
+            const int64_t off = u_tap + 16 * u_icg;
 #pragma unroll
-        for (int c = 0; c < KC; ++c) {
-            uint8_t* const st = sT + slot * STAGE + c * CHUNK + wave * 1024;
-#pragma unroll
-            for (int i = 0; i < NA; ++i)
-                load_to_lds_16(wsrc[i] + w_off + 64 * c, st + NW * i * 1024);
+            for (int i = 0; i < NA; ++i) load_to_lds_16(real ? wbase + woff[i] + 16 * u : wzero, st + NW * i * 1024);
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
-                const uint8_t* src = bsrc[i] + it_off + 64 * c;
-                if (!w.inside) src = ((rows[i] >> it_ky) & (cols[i] >> it_kx) & 1u) ? src : fillp;
-                load_to_lds_16(src, st + (ABLK + NW * i) * 1024);
+                const bool ok = real && ((taps[i] >> u_ky) & (taps[i] >> (16 + u_kx)) & 1u) != 0;
+                load_to_lds_16(ok ? bsrc[i] + off : fillp, st + (BN / 8 + NW * i) * 1024);
             }
-        }
-        w_off += 64 * KC;
-        it_off += 64 * KC;
-        it_c64 += KC;
-        if (it_c64 == w.nc64) {
-            it_c64 = 0;
-            tap_off += a.in_sw;
-            if (++it_kx == a.KX) {
-                it_kx = 0;
-                ++it_ky;
-                tap_off += w.row_adv;
+            u += 8;
+            u_icg += 8;
+            wrap_unit();
+        } else {
+#pragma unroll
+            for (int i = 0; i < NA; ++i) load_to_lds_16(it_w, woff[i], st + NW * i * 1024);
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const bool ok = ((taps[i] >> it_ky) & (taps[i] >> (16 + it_kx)) & 1u) != 0;
+                load_to_lds_16(ok ? bsrc[i] + it_off : fillp, st + (BN / 8 + NW * i) * 1024);
             }
-            it_off = tap_off;
+            it_w += 128;
+            it_off += 128;
+            if (++it_c == w.nc128) {
+                it_c = 0;
+                tap_off += a.in_sw;
+                if (++it_kx == a.KX) {
+                    it_kx = 0;
+                    ++it_ky;
+                    tap_off += w.row_adv;
+                }
+                it_off = tap_off;
+            }
         }
     };
 
     const int S = w.nsteps;
-    __syncthreads();  // (sOutOff, sWsum, sFlags are in place; no full barrier until the reduction is over)
-    // NS - 1 steps in flight before the first is consumed.
 #pragma unroll
-    for (int j = 0; j < NS - 1; ++j) {
+    for (int j = 0; j < NS; ++j)
         if (j < S) request(j);
-    }
     // the table rows of the workgroup's channels travel while the first operands do
     int32_t tw2 = 0, tbias = 0;
     if (tid < noc) {
@@ -175,62 +221,104 @@ __global__ __launch_bounds__(64 * WM * WN, tiled_min_waves(WM * WN, TM * TN)) vo
         tbias = trow[3];
     }
 
-    // operand reads: lane (c16, q) reads row c16 of a fragment, piece q
-    const int frag_off = c16 * 64 + (((lane >> 4) ^ swz(c16)) << 4);
-    const int a_rd = (wn * TN) * 1024 + frag_off;
-    const int b_rd = BN * 64 + (wm * TM) * 1024 + frag_off;
+    // operand reads: lane (c16, q) reads row c16 of a fragment, piece q of half 0; half 1 is at the address with bit 6 flipped
+    const int frag0 = c16 * 128 + (((lane >> 4) ^ swz8(c16 >> 1)) << 4);
+    const int a_rd = (wn * TN) * 2048;
+    const int b_rd = BN * 128 + (wm * TM) * 2048;
 
     v4i acc[TN][TM];
-    v4i wsa[TN];  // weight sums (input zero point away from the storage offset only)
+    constexpr int NWS = (TN + WM - 1) / WM;
+    v4i wsa[NWS];  // sums of this wave's share of the weight fragments (input zero point away from the storage offset only)
+    v4i asum[TM];  // ASUM: sums of the pixel fragments
 #pragma unroll
-    for (int f = 0; f < TN; ++f) {
-        wsa[f] = v4i{0, 0, 0, 0};
+    for (int f = 0; f < TN; ++f)
 #pragma unroll
         for (int x = 0; x < TM; ++x) acc[f][x] = v4i{0, 0, 0, 0};
-    }
+#pragma unroll
+    for (int x = 0; x < TM; ++x) asum[x] = v4i{0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < NWS; ++i) wsa[i] = v4i{0, 0, 0, 0};
     const int axor = (int)a.a_xor, wxor = (int)a.w_xor;
     const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
 
     // The reduction loop, compiled twice: with and without the weight sums.
     auto reduce = [&](auto with_sums) {
         constexpr bool WS = decltype(with_sums)::value;
-        int slot = 0;  // ring slot of step s
-        for (int s = 0; s < S; ++s) {
-            // The requests of step s are this wave's oldest; younger ones (at most NS - 2 steps) may stay in flight.
-            // Near the end fewer are younger, so there everything is waited for.
-            if (s + NS - 1 <= S) __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 2) * (NA + NB) * KC));
-            else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-            // Every wave's pieces of step s are in LDS, and every wave has left step s - 1's slot. (The bare barrier:
-            // __syncthreads() would first wait for ALL outstanding loads, which empties the ring at every step.)
-            __builtin_amdgcn_s_barrier();
-            if (s + NS - 1 < S) request(slot == 0 ? NS - 1 : slot - 1);
-            const uint8_t* const st = sT + slot * STAGE;
-            v4i fa[KC][TN], fb[KC][TM];
+        constexpr int R = TN + TM, G = TM > 1 ? TM - 1 : 1;  // operand reads of a half step, groups that carry them
+        v4i fa[2][TN], fb[2][TM];
+        auto read = [&](const uint8_t* st, int i, auto par) {  // par: half of the step, and register set
+            constexpr int P = decltype(par)::value;
+            const uint8_t* const at = st + (frag0 ^ (64 * P));
+            if (i < TN) fa[P][i] = *reinterpret_cast<const v4i*>(at + a_rd + i * 2048);
+            else fb[P][i - TN] = *reinterpret_cast<const v4i*>(at + b_rd + (i - TN) * 2048);
+        };
+        auto prepare_next = [&](auto par) {
+            constexpr int P = decltype(par)::value;
+            if (wxor != 0) {  // uniform
 #pragma unroll
-            for (int c = 0; c < KC; ++c) {
-#pragma unroll
-                for (int f = 0; f < TN; ++f) fa[c][f] = *reinterpret_cast<const v4i*>(st + c * CHUNK + a_rd + f * 1024);
-#pragma unroll
-                for (int x = 0; x < TM; ++x) fb[c][x] = *reinterpret_cast<const v4i*>(st + c * CHUNK + b_rd + x * 1024);
+                for (int f = 0; f < TN; ++f) fa[P][f] ^= wxor;
             }
+            fb[P][0] ^= axor;
+        };
+        // One half step from the registers of set P, while the operands of the next half are read from ring slot `next` into the
+        // other set; req() issues requests.
+        auto half = [&](const uint8_t* next, auto par, auto&& req) {
+            constexpr int P = decltype(par)::value;
+            const auto other = std::integral_constant<int, P ^ 1>{};
 #pragma unroll
-            for (int c = 0; c < KC; ++c) {
-                if (wxor != 0) {  // uniform
+            for (int x = 0; x < TM; ++x) {
 #pragma unroll
-                    for (int f = 0; f < TN; ++f) fa[c][f] ^= wxor;
-                }
-#pragma unroll
-                for (int x = 0; x < TM; ++x) fb[c][x] ^= axor;
-#pragma unroll
-                for (int f = 0; f < TN; ++f)
-#pragma unroll
-                    for (int x = 0; x < TM; ++x) acc[f][x] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[c][f], fb[c][x], acc[f][x], 0, 0, 0);
+                for (int f = 0; f < TN; ++f) acc[f][x] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[P][f], fb[P][x], acc[f][x], 0, 0, 0);
                 if constexpr (WS) {
+                    if (x == 0) {
 #pragma unroll
-                    for (int f = 0; f < TN; ++f) wsa[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[c][f], ones, wsa[f], 0, 0, 0);
+                        for (int f = 0; f < TN; ++f)
+                            if (f % WM == wm) wsa[f / WM] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[P][f], ones, wsa[f / WM], 0, 0, 0);
+                    }
+                }
+                if constexpr (ASUM) asum[x] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, fb[P][x], asum[x], 0, 0, 0);
+                if (x + 1 < TM) fb[P][x + 1] ^= axor;
+#pragma unroll
+                for (int i = 0; i < R; ++i)
+                    if (i * G / R == x) read(next, i, other);
+                if (x + 1 == TM) prepare_next(other);
+#pragma unroll
+                for (int g = 0; g < TN; ++g) {  // one matrix instruction, one vector instruction, and an LDS read behind the first two
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x2, 1, 0);
+                    if (g < 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                if (x == 0) {
+                    req();
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
-            slot = slot == NS - 1 ? 0 : slot + 1;
+        };
+        const auto P0 = std::integral_constant<int, 0>{};
+        const auto P1 = std::integral_constant<int, 1>{};
+        if (S >= NS) __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 1) * (NA + NB)));
+        else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        warm.release();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < R; ++i) read(sT, i, P0);
+        prepare_next(P0);
+        for (int s = 0; s < S; ++s) {
+            const int slot = (int)((uint32_t)s % NS), next = (int)((uint32_t)(s + 1) % NS);
+            half(sT + slot * STAGE, P0, [] {});
+            // Step s + 1 has to be in LDS before it is read: the requests up to step s + NS - 1 are out, those younger than step
+            // s + 1 may stay in flight. Every wave holds step s in registers before its slot is requested again.
+            if (s + NS <= S) __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 2) * (NA + NB)));
+            else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            // (the bare barrier: __syncthreads() would first wait for all outstanding loads)
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            // (the last step reads a slot that holds nothing of use)
+            half(sT + next * STAGE, P1, [&] { if (s + NS < S) request(slot); });
         }
     };
     if (a.da != 0) reduce(std::true_type{});
@@ -238,12 +326,16 @@ __global__ __launch_bounds__(64 * WM * WN, tiled_min_waves(WM * WN, TM * TN)) vo
     __syncthreads();
 
     // ---- per-channel constants (thread = channel), as in the weights-resident kernel -----------------------
-    if (a.da != 0 && wm == 0 && c16 == 0) {
+    if (a.da != 0 && c16 == 0) {
         // every column of a sum fragment holds the same sums: lane (0, q) publishes rows 4q .. 4q + 3
 #pragma unroll
-        for (int f = 0; f < TN; ++f)
+        for (int i = 0; i < NWS; ++i) {
+            const int f = WM * i + wm;
+            if (f < TN) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) sWsum[wn * CW + channel_of_frag_row<TN>(f, 4 * (lane >> 4) + r)] = wsa[f][r];
+                for (int r = 0; r < 4; ++r) sWsum[wn * CW + channel_of_frag_row<TN>(f, 4 * (lane >> 4) + r)] = wsa[i][r];
+            }
+        }
     }
     const int64_t acc_bound = min((int64_t)a.ktot * 65025, (int64_t)2147483648LL);
     if (tid < BN) {
@@ -283,7 +375,8 @@ __global__ __launch_bounds__(64 * WM * WN, tiled_min_waves(WM * WN, TM * TN)) vo
     }
     if (tid < BN) {
         const int32_t mult = table_mult(tw2), shift = table_shift(tw2);
-        const int32_t corr = a.da * sWsum[tid];  // |da| <= 255, |sum w'| < 2^23
+        // |da| <= 255, |sum w'| < 2^23; with a weight zero-point offset the constant term of the whole (padded) reduction joins
+        const int32_t corr = a.da * sWsum[tid] + (ASUM ? w.nsteps * 128 * a.da * a.dw : 0);
         const double M = ppe_scale_M(mult, shift);
         double B = __builtin_fma((double)corr, M, ppe_scale_B(tbias, M, shift, a.ppe.round_mode));
         if (pmode != PPE_MODE_INT) B += ep.zp_fold;  // floor(x + zp) = floor(x) + zp
@@ -313,89 +406,104 @@ __global__ __launch_bounds__(64 * WM * WN, tiled_min_waves(WM * WN, TM * TN)) vo
         const int r = (wm * TM + x) * 16 + c16;
         valid[x] = m0 + r < a.M;
         dst[x] = a.out + sOutOff[r] + (int64_t)(oc0 + wn * CW) * a.out_sc;
-        dws[x] = 0;
+        dws[x] = ASUM ? a.dw * asum[x][0] : 0;  // (every row of a sum fragment is the pixel's sum)
     }
     const int q = lane >> 4;
     const int nocw = noc - wn * CW;
     const EpiSmem ew = {sM + wn * CW, nullptr, sW2 + wn * CW, sBias + wn * CW, nullptr, nullptr};
     const double* const bw = sBfull + wn * CW;
     const int32_t* const cw = sCorr + wn * CW;
-    uint4 other[FZ ? TM : 1];
-    if constexpr (FZ) {
-        if (nocw > 0) {  // uniform per wave; lanes past the last channel read a duplicate inside the tensor
-            const int ch0 = min(16 * q, nocw - 16);
+    // (at most EX pixel fragments at a time: over more of them the epilogue's state does not fit beside the accumulators)
+    constexpr int EX = TM > 4 ? 2 : TM;
+    static_assert(TM == EX || TM == 4 * EX, "epilogue rounds");
+    const auto epilogue = [&](auto first) {
+        constexpr int x0 = decltype(first)::value;
+        v4i ax[TN][EX];
+        uint8_t* dx[EX];
+        bool vx[EX];
+        int32_t wx[EX];
+        uint4 other[FZ ? EX : 1];
 #pragma unroll
-            for (int x = 0; x < TM; ++x) other[x] = *reinterpret_cast<const uint4*>(w.fz.other + ((dst[x] + ch0) - a.out));
+        for (int x = 0; x < EX; ++x) {
+#pragma unroll
+            for (int f = 0; f < TN; ++f) ax[f][x] = acc[f][x0 + x];
+            dx[x] = dst[x0 + x];
+            vx[x] = valid[x0 + x];
+            wx[x] = dws[x0 + x];
         }
+        if constexpr (FZ) {
+            if (nocw > 0) {  // uniform per wave; lanes past the last channel read a duplicate inside the tensor
+                const int ch0 = min(16 * q, nocw - 16);
+#pragma unroll
+                for (int x = 0; x < EX; ++x) other[x] = *reinterpret_cast<const uint4*>(w.fz.other + ((dx[x] + ch0) - a.out));
+            }
+        }
+        if (pmode == PPE_MODE_HI) wres_epilogue<TN, EX, PPE_MODE_HI, FZ>(a, ew, bw, cw, ax, wx, q, nocw, dx, vx, pu, ep, &w.fz, other);
+        else if (pmode == PPE_MODE_HI_SLOPE) wres_epilogue<TN, EX, PPE_MODE_HI_SLOPE, FZ>(a, ew, bw, cw, ax, wx, q, nocw, dx, vx, pu, ep, &w.fz, other);
+        else if (pmode == PPE_MODE_FOLDED) wres_epilogue<TN, EX, PPE_MODE_FOLDED, FZ>(a, ew, bw, cw, ax, wx, q, nocw, dx, vx, pu, ep, &w.fz, other);
+        else if (pmode == PPE_MODE_SLOPE) wres_epilogue<TN, EX, PPE_MODE_SLOPE, FZ>(a, ew, bw, cw, ax, wx, q, nocw, dx, vx, pu, ep, &w.fz, other);
+        else wres_epilogue<TN, EX, PPE_MODE_INT, FZ>(a, ew, bw, cw, ax, wx, q, nocw, dx, vx, pu, ep, &w.fz, other);
+    };
+    epilogue(std::integral_constant<int, 0>{});
+    if constexpr (TM > EX) {
+        epilogue(std::integral_constant<int, EX>{});
+        epilogue(std::integral_constant<int, 2 * EX>{});
+        epilogue(std::integral_constant<int, 3 * EX>{});
     }
-    if (pmode == PPE_MODE_HI) wres_epilogue<TN, TM, PPE_MODE_HI, FZ>(a, ew, bw, cw, acc, dws, q, nocw, dst, valid, pu, ep, &w.fz, other);
-    else if (pmode == PPE_MODE_HI_SLOPE) wres_epilogue<TN, TM, PPE_MODE_HI_SLOPE, FZ>(a, ew, bw, cw, acc, dws, q, nocw, dst, valid, pu, ep, &w.fz, other);
-    else if (pmode == PPE_MODE_FOLDED) wres_epilogue<TN, TM, PPE_MODE_FOLDED, FZ>(a, ew, bw, cw, acc, dws, q, nocw, dst, valid, pu, ep, &w.fz, other);
-    else if (pmode == PPE_MODE_SLOPE) wres_epilogue<TN, TM, PPE_MODE_SLOPE, FZ>(a, ew, bw, cw, acc, dws, q, nocw, dst, valid, pu, ep, &w.fz, other);
-    else wres_epilogue<TN, TM, PPE_MODE_INT, FZ>(a, ew, bw, cw, acc, dws, q, nocw, dst, valid, pu, ep, &w.fz, other);
 }
 
-template <int WM, int WN, int TM, int TN, int NS, int KC = 1>
+template <int WM, int WN, int TM, int TN, int NS, int OCC>
 hipError_t launch_shape(TiledArgs& w, bool fused, hipStream_t stream) {
     constexpr int BM = 16 * TM * WM;
     constexpr int BN = 16 * TN * WN;
-    constexpr size_t lds = (size_t)NS * (BM + BN) * 64 * KC;
+    constexpr size_t lds = (size_t)NS * (BM + BN) * 128;
     const ConvArgs& a = w.a;
-    if (w.nc64 % KC != 0) return hipErrorNotSupported;
-    w.nsteps = a.KY * a.KX * (w.nc64 / KC);
     w.ntm = (uint32_t)(((int64_t)a.M + BM - 1) / BM);
     w.ntn = (uint32_t)((a.bc + BN - 1) / BN);
-    const uint64_t total = (uint64_t)w.ntm * w.ntn;
-    if (total > 0x7ffffff0ull) return hipErrorNotSupported;
-    const dim3 grid(xcd_grid((uint32_t)total)), block(64 * WM * WN);
-    if (fused) {
-        if constexpr (TN == 4) {
-            auto kernel = &conv_tiled_kernel<WM, WN, TM, TN, NS, KC, true>;
-            static LdsGrant grant;
-            if (const hipError_t e = grant.ensure(reinterpret_cast<const void*>(kernel), lds, 48 * 1024); e != hipSuccess) return e;
-            return emit(kernel, grid, block, lds, stream, w);
-        }
-        return hipErrorNotSupported;
-    }
-    auto kernel = &conv_tiled_kernel<WM, WN, TM, TN, NS, KC, false>;
-    static LdsGrant grant;
-    if (const hipError_t e = grant.ensure(reinterpret_cast<const void*>(kernel), lds, 48 * 1024); e != hipSuccess) return e;
-    return emit(kernel, grid, block, lds, stream, w);
+    w.div_ntn = make_fastdiv(w.ntn);
+    w.warm = make_warm(a.w + (int64_t)a.z0 * a.w_soc, (int64_t)a.bc * a.w_soc, std::min<int64_t>(xcd_grid(w.ntm * w.ntn) / kNumXcd, 32 * 4 * OCC / (WM * WN)) * (WM * WN));
+    if ((uint64_t)w.ntm * w.ntn > 0x7ffffff0ull) return hipErrorNotSupported;
+    const auto go = [&](auto kernel, LdsGrant& grant) {
+        if (const hipError_t e = grant.ensure(reinterpret_cast<const void*>(kernel), lds, 48 * 1024); e != hipSuccess) return e;
+        return emit(kernel, dim3(xcd_grid(w.ntm * w.ntn)), dim3(64 * WM * WN), lds, stream, w);
+    };
+    static LdsGrant grants[4];
+    if (a.dw != 0) return fused ? hipErrorNotSupported : go(&conv_tiled_kernel<WM, WN, TM, TN, NS, OCC, false, TILED_UNITS_ASUM>, grants[0]);
+    if (a.IC % 128 != 0) return fused ? hipErrorNotSupported : go(&conv_tiled_kernel<WM, WN, TM, TN, NS, OCC, false, TILED_UNITS>, grants[1]);
+    if (!fused) return go(&conv_tiled_kernel<WM, WN, TM, TN, NS, OCC, false, TILED_CHUNKS>, grants[2]);
+    if constexpr (TN == 4) return go(&conv_tiled_kernel<WM, WN, TM, TN, NS, OCC, true, TILED_CHUNKS>, grants[3]);
+    return hipErrorNotSupported;
 }
 
 }  // namespace
 
-// Shapes: 1 = 128 px x 128 ch (4 waves), 2 = 64 px x 128 ch (4 waves), 3 = 256 px x 128 ch (8 waves),
-// 4 = 128 px x 64 ch (4 waves), 5 = shape 1 with steps of 128 bytes of the reduction (input channels a multiple of 128),
-// 6 = shape 5 as eight waves of 32 px x 64 ch, two workgroups = sixteen waves per CU. shape 0 = automatic.
+// Shapes (pixels x channels): 1 = 256 x 256, 2 = 256 x 128, 3 = 128 x 128 (eight waves each), 4 = 128 x 64, 5 = 64 x 128,
+// 6 = 64 x 64, 7 = 256 x 64 (four waves).
 hipError_t launch_conv_tiled(const ConvArgs& a, hipStream_t stream, int shape, const FuseAdd* fuse) {
-    if (a.IC % 64 != 0 || a.dw != 0 || a.KY > 32 || a.KX > 32) return hipErrorNotSupported;
+    if (a.KY > 15 || a.KX > 15) return hipErrorNotSupported;
     if (a.M > 0x7fffffff - 1024) return hipErrorNotSupported;
     if (fuse != nullptr && a.out_sc != 1) return hipErrorNotSupported;
+    if (a.w_soc > 0x7fffffffLL / 256) return hipErrorNotSupported;  // (32-bit offsets within a tile's weights)
+    // (weight zero-point offset: the activation sums times dw and the constant stay inside int32)
+    if (a.dw != 0 && ((int64_t)a.ktot + 128) * 255 * 255 > 0x7fffffffLL) return hipErrorNotSupported;
     TiledArgs w;
     memset(&w, 0, sizeof(w));
     w.a = a;
     w.a.fill_raw = (a.fill ^ a.a_xor) & 0xFFu;
     if (fuse) w.fz = *fuse;
-    w.nc64 = a.IC / 64;
-    w.nsteps = a.KY * a.KX * w.nc64;
+    w.nc128 = a.IC / 128;
+    w.wraps = (a.ICG + 7) / a.ICG;
+    w.nsteps = (a.KG + 7) / 8;
     w.row_adv = a.in_sh - (int64_t)a.KX * a.in_sw;
-    const int64_t iy_lo = (int64_t)a.y0 * a.SY - a.PT, iy_hi = (int64_t)(a.y0 + a.bh - 1) * a.SY - a.PT + a.KY - 1;
-    const int64_t ix_lo = (int64_t)a.x0 * a.SX - a.PL, ix_hi = (int64_t)(a.x0 + a.bw - 1) * a.SX - a.PL + a.KX - 1;
-    w.inside = iy_lo >= 0 && iy_hi < a.H && ix_lo >= 0 && ix_hi < a.W;
-    if (shape == 0) {
-        // The largest tile that still gives every CU about two workgroups.
-        const auto groups = [&](int bm, int bn) { return (((int64_t)a.M + bm - 1) / bm) * ((a.bc + bn - 1) / bn); };
-        shape = groups(128, 128) >= 512 ? (a.IC % 128 == 0 ? 6 : 1) : 2;
-    }
     const bool fz = fuse != nullptr;
     switch (shape) {
-    case 1: return launch_shape<2, 2, 4, 4, 4>(w, fz, stream);
-    case 2: return launch_shape<2, 2, 2, 4, 4>(w, fz, stream);
-    case 3: return launch_shape<4, 2, 4, 4, 3>(w, fz, stream);
-    case 4: return launch_shape<2, 2, 4, 2, 4>(w, fz, stream);
-    case 5: return launch_shape<2, 2, 4, 4, 2, 2>(w, fz, stream);
-    case 6: return launch_shape<4, 2, 2, 4, 2, 2>(w, fz, stream);
+    case 1: return launch_shape<2, 4, 8, 4, 2, 2>(w, fz, stream);
+    case 2: return launch_shape<4, 2, 4, 4, 2, 2>(w, fz, stream);
+    case 3: return launch_shape<4, 2, 2, 4, 2, 4>(w, fz, stream);
+    case 4: return launch_shape<4, 1, 2, 4, 2, 3>(w, fz, stream);
+    case 5: return launch_shape<2, 2, 2, 4, 2, 3>(w, fz, stream);
+    case 6: return launch_shape<4, 1, 1, 4, 2, 4>(w, fz, stream);
+    case 7: return launch_shape<4, 1, 4, 4, 2, 2>(w, fz, stream);
     default: return hipErrorNotSupported;
     }
 }

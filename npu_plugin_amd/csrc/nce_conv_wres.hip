@@ -1093,6 +1093,45 @@ extern "C" void nceProbeSetWresTrace(uint64_t* device_buffer) {
     g_wres_trace_seq = 0;
 }
 #endif
+// Tiles per workgroup: one workgroup per CU where the tiles reach that far (the waves of a workgroup then take unequal
+// numbers of tiles, which costs less than leaving CUs idle or queueing a second round).
+static int64_t wres_tiles_per_group(const ConvArgs& a, int nf, int bf, int nwaves) {
+    const int cus = tls_launch.per_xcd ? 32 : 256;
+    const int64_t ntiles = ((int64_t)a.M + 16 * bf - 1) / (16 * bf);
+    const int64_t slices = (a.bc + 16 * nf - 1) / (16 * nf);
+    const int64_t groups = std::max<int64_t>(1, cus / slices);
+    return std::max<int64_t>(nwaves, (ntiles + groups - 1) / groups);
+}
+
+WresShape wres_shape_for(const ConvArgs& a, bool fused) {
+    const int nsteps = (a.KG + 3) / 4, ntaps = a.KY * a.KX;
+    const size_t wl4 = (size_t)((nsteps + 1) / 2 * 2) * 4 * 1024, wl2 = wl4 / 2;  // with the padding step
+    WresShape s = {};
+    s.ok = wl2 <= kWresLdsCap - (a.IC % 64 != 0 ? 4096 : 0) && !(a.IC % 64 == 0 && ntaps > 31);
+    // Measured over the ResNet-50 layer shapes, the best shape is always the LARGEST tile that still yields about 1500 wave
+    // tiles (six waves per CU, one round of workgroups); beyond that, waves take several tiles each rather than the grid
+    // growing.
+    auto wave_tiles = [&](int nf, int bf) {
+        return (((int64_t)a.M + 16 * bf - 1) / (16 * bf)) * ((a.bc + 16 * nf - 1) / (16 * nf));
+    };
+    const bool nf4_ok = wl4 <= kWresLdsCap && a.bc > 32;
+    // (1x1 kernels over more than 64 input channels: measured faster with smaller pixel tiles, about 24 per CU)
+    // (per-XCD form: an eighth of the work on an eighth of the CUs - the same choices as for the whole task)
+    const int cus = tls_launch.per_xcd ? 32 : 256;
+    const int64_t want = ((ntaps == 1 && nsteps > 1) ? 6000 : 1500) * cus / 256;
+    // (per-XCD form: tiles of at most 32 pixels - the persistent kernel carries no 64-pixel instantiation, whose registers
+    // every layer's path would pay for)
+    s.nf = nf4_ok ? 4 : 2;
+    s.bf = tls_launch.per_xcd ? 2 : 4;
+    while (s.bf > 1 && wave_tiles(s.nf, s.bf) < want) s.bf >>= 1;
+    if (s.nf == 4 && wave_tiles(s.nf, s.bf) < 1500 * cus / 256) s.nf = 2;
+    if (fused && nf4_ok) s.nf = 4;
+    s.tiles_per_group = wres_tiles_per_group(a, s.nf, s.bf, 8);
+    s.slices = (a.bc + 16 * s.nf - 1) / (16 * s.nf);
+    s.groups = (((int64_t)a.M + 16 * s.bf - 1) / (16 * s.bf) + s.tiles_per_group - 1) / s.tiles_per_group;
+    return s;
+}
+
 hipError_t launch_conv_wres(const ConvArgs& a, hipStream_t stream, bool allow_chunked, const FuseAdd* fuse) {
     if (a.KY > 32 || a.KX > 32) return hipErrorNotSupported;
     // (pixel indices of tiles past the end - waves without a tile still form addresses - must stay below 2^31)
@@ -1135,33 +1174,10 @@ hipError_t launch_conv_wres(const ConvArgs& a, hipStream_t stream, bool allow_ch
     // one bit per tap, bit 31 stays clear; larger kernels take the chunked kernel's row / column bits
     if (mode == WRES_FAST_MASK && a.KY * a.KX > 31) return allow_chunked && !w.fused ? launch_conv_wres_chunked(w, stream) : hipErrorNotSupported;
 
-    // Shape of the work: nf channel fragments per slice, bf pixel fragments per wave tile. Measured on
-    // MI355X over the ResNet-50 layer shapes, the best shape is always the LARGEST tile that still
-    // yields about 1500 wave tiles (six waves per CU, one round of workgroups); beyond that, waves take
-    // several tiles each rather than the grid growing.
-    auto wave_tiles = [&](int nf, int bf) {
-        return (((int64_t)a.M + 16 * bf - 1) / (16 * bf)) * ((a.bc + 16 * nf - 1) / (16 * nf));
-    };
-    const bool nf4_ok = wl4 <= kWresLdsCap && a.bc > 32;
-    // (1x1 kernels over more than 64 input channels: measured faster with smaller pixel tiles, about 24 per CU)
-    // (per-XCD form: an eighth of the work on an eighth of the CUs - the same choices as for the whole task)
-    const int cus = tls_launch.per_xcd ? 32 : 256;
-    const int64_t want = ((w.ntaps == 1 && w.nsteps > 1) ? 6000 : 1500) * cus / 256;
-    // (per-XCD form: tiles of at most 32 pixels - the persistent kernel carries no 64-pixel instantiation, whose registers
-    // every layer's path would pay for)
-    int nf = nf4_ok ? 4 : 2, bf = tls_launch.per_xcd ? 2 : 4;
-    while (bf > 1 && wave_tiles(nf, bf) < want) bf >>= 1;
-    if (nf == 4 && wave_tiles(nf, bf) < 1500 * cus / 256) nf = 2;
+    const WresShape shape = wres_shape_for(a, w.fused != 0);
+    int nf = shape.nf, bf = shape.bf;
     const int nwaves = 8;
     int tpw = 1;
-    // Tiles per workgroup: one workgroup per CU where the tiles reach that far (the waves of a workgroup then
-    // take unequal numbers of tiles, which costs less than leaving CUs idle or queueing a second round).
-    const auto pick_tpg = [&](int nf_, int bf_, int nw_) {
-        const int64_t ntiles = ((int64_t)a.M + 16 * bf_ - 1) / (16 * bf_);
-        const int64_t slices = (a.bc + 16 * nf_ - 1) / (16 * nf_);
-        const int64_t groups = std::max<int64_t>(1, cus / slices);
-        return (uint32_t)std::max<int64_t>(nw_, (ntiles + groups - 1) / groups);
-    };
 
     int nw = nwaves;
     bool forced_tpw = false;
@@ -1172,8 +1188,8 @@ hipError_t launch_conv_wres(const ConvArgs& a, hipStream_t stream, bool allow_ch
         if (fnw >= 1 && fnw <= 8) nw = fnw;
         if (ftpw >= 1) tpw = ftpw, forced_tpw = true;  // (0: keep the automatic choice below)
     }
-    if (w.fused && nf4_ok) nf = 4;  // (the fused add exists for the 64-channel kernels)
-    w.tpg = forced_tpw ? 0 : pick_tpg(nf, bf, nw);
+    if (w.fused && wl4 <= kWresLdsCap && a.bc > 32) nf = 4;  // (the fused add exists for the 64-channel kernels)
+    w.tpg = forced_tpw ? 0 : (int32_t)wres_tiles_per_group(a, nf, bf, nw);
     if (nf == 4) return launch_wres_nf4(w, bf, mode, nw, tpw, stream);
     return launch_bf<2>(w, bf, mode, nw, tpw, stream);
 }
