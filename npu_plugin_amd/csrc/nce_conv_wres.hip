@@ -1124,6 +1124,10 @@ WresShape wres_shape_for(const ConvArgs& a, bool fused) {
     s.nf = nf4_ok ? 4 : 2;
     s.bf = tls_launch.per_xcd ? 2 : 4;
     while (s.bf > 1 && wave_tiles(s.nf, s.bf) < want) s.bf >>= 1;
+    // (one reduction step, per-lane loads, five slices and more: of 11 such tasks from 20,000 to 350,000 pixels tiles of 32 pixels
+    // were 10-39 % ahead of 64 in all - 1x1 over 48 channels to 288, 28768 pixels: 11.6 us with 64, 8.4 us with 32, 8.7 us with 16.
+    // Up to four slices and from two steps on it is the other way round, by 2-58 %.)
+    if (a.IC % 64 != 0 && nsteps == 1 && s.nf == 4 && a.bc > 256 && s.bf > 2) s.bf = 2;
     if (s.nf == 4 && wave_tiles(s.nf, s.bf) < 1500 * cus / 256) s.nf = 2;
     if (fused && nf4_ok) s.nf = 4;
     s.tiles_per_group = wres_tiles_per_group(a, s.nf, s.bf, 8);
