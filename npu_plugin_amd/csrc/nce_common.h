@@ -168,6 +168,7 @@ struct Options {
     int persistent = 0;       // NCE_HIP_PERSISTENT: task lists run runs of weights-resident convolutions as one persistent launch
     int persistent_wait_us = 2000000;  // NCE_HIP_PERSISTENT_WAIT_US: time after which a persistent launch's waits give up
     int tiled = -1;           // NCE_HIP_CONV_TILED: -1 automatic, 0 never, 1.. force that shape of the LDS-tiled kernel
+    int band = -1;            // NCE_HIP_CONV_BAND: -1 automatic, 0 never, 1 .. 4: that run length of the band kernel
     int split = -1;           // NCE_HIP_CONV_SPLIT: -1 automatic, 0 never, 1.. force that tile of the split-reduction kernel
     int patch = -1;           // NCE_HIP_CONV_PATCH: -1 automatic, 0 never, 1 = wherever its conditions hold; "nf,pr[,waves]" also forces its shape
     int patch_nf = 0, patch_pr = 0, patch_waves = 0, patch_npx = 0;

@@ -390,15 +390,36 @@ static double estimate_wres(const ConvArgs& a, const WresShape& s) {
            (a.bc % 64 != 0 ? 0.2556 * out : 0.0);
 }
 
+// (fitted the same way on 272 tasks with kernels larger than 1x1 over ragged channel counts, 1 to 128 images, every run length
+// forced: within 8 % of the measured time for nine tasks in ten)
+static double estimate_band(const ConvArgs& a, int shape) {
+    struct Run {
+        double base, run, step, stage, first, out, wsum, asum, fresh;
+    };
+    static const Run runs[4] = {
+        {3.696, 0.9364, 0.0665, 0.0313, 0.1163, 0.3344, 0.0302, 0.0077, 0.0921},
+        {3.523, 1.422, 0.0557, 0.0477, 0.154, 0.2005, 0.0284, 0.0455, 0.1811},
+        {3.999, 1.4983, 0.0461, 0.0569, 0.1825, 0.1735, 0.0287, 0.0479, 0.3389},
+        {4.967, 1.3452, 0.0, 0.0885, 0.2137, 0.2405, 0.0216, 0.0813, 0.4274},
+    };
+    const Run& t = runs[shape - 1];
+    const BandShape b = band_shape_for(a, shape);
+    if (!b.ok) return 1e30;
+    const double steps = (double)((a.KG + 3) / 4), rounds = (double)((b.groups + 255) / 256), n = (double)b.tpg * rounds;
+    return t.base + t.run * n + t.step * n * steps + t.stage * steps * b.nf * rounds + t.first * (double)b.first_passes + 1e-6 * t.out * (double)a.M * a.bc +
+           (a.da != 0 ? t.wsum * steps : 0.0) + (a.dw != 0 ? t.asum * n * steps : 0.0) + t.fresh * (double)b.fresh_passes * n;
+}
+
 struct ConvChoice {
-    int split, tiled;  // the tile of the split-reduction / LDS-tiled kernel to try first; 0, 0: the other kernels
+    int split, tiled, band;  // the tile of the split-reduction / LDS-tiled / band kernel to try first; all 0: the other kernels
 };
 static ConvChoice choose_conv(const ConvArgs& a, bool fused) {
-    if (tls_launch.per_xcd || options().conv_path != 0 || options().wres_forced) return {0, 0};
-    if (options().split > 0) return {options().split, 0};
-    if (options().tiled > 0) return {0, options().tiled};
-    if (options().patch > 0) return {0, 0};
-    ConvChoice c = {0, 0};
+    if (tls_launch.per_xcd || options().conv_path != 0 || options().wres_forced) return {0, 0, 0};
+    if (options().split > 0) return {options().split, 0, 0};
+    if (options().tiled > 0) return {0, options().tiled, 0};
+    if (options().patch > 0) return {0, 0, 0};
+    if (options().band > 0) return {0, 0, options().band};
+    ConvChoice c = {0, 0, 0};
     const WresShape s = wres_shape_for(a, fused);
     // (The weights-resident kernel's estimate is the least certain: it has to be beaten by 10 %. Of the 734 tasks four then come
     // out more than 4 % slower than it. Those were tasks enqueued again and again, whose weights sit in L2. In a list they come
@@ -410,10 +431,14 @@ static ConvChoice choose_conv(const ConvArgs& a, bool fused) {
     double best = !fused && patch_wanted(a) ? 0.0 : s.ok && (!fused || s.nf == 4) ? wres_factor * estimate_wres(a, s) : 1e30;
     if (options().split < 0)
         for (int i = 1; i <= 5; ++i)
-            if (const double t = estimate_split(a, i); t < best) best = t, c = {i, 0};
+            if (const double t = estimate_split(a, i); t < best) best = t, c = {i, 0, 0};
     if (options().tiled < 0 && !(fused && (a.IC % 128 != 0 || a.dw != 0)))
         for (int i = fused ? 2 : 1; i <= 7; ++i)  // (256 x 256 tiles, one workgroup per CU, leave an add's traffic with nothing beside it)
-            if (const double t = estimate_tiled(a, i); t < best) best = t, c = {0, i};
+            if (const double t = estimate_tiled(a, i); t < best) best = t, c = {0, i, 0};
+    // (a 1x1 kernel has no rows to share between taps; whole 64-channel pixels are read as they are by the kernels above)
+    if (options().band < 0 && !fused && a.KY * a.KX > 1 && a.IC % 64 != 0)
+        for (int i = 1; i <= 4; ++i)
+            if (const double t = estimate_band(a, i); t < best) best = t, c = {0, 0, i};
     return c;
 }
 
@@ -475,6 +500,8 @@ hipError_t launch_conv(const TaskDev& t, const Box& box, hipStream_t stream) {
     if (choice.split != 0) e = launch_conv_split(a, stream, choice.split);
     if (e != hipErrorNotSupported) return e;
     if (choice.tiled != 0) e = launch_conv_tiled(a, stream, choice.tiled);
+    if (e != hipErrorNotSupported) return e;
+    if (choice.band != 0) e = launch_conv_band(a, stream, choice.band);
     if (e != hipErrorNotSupported) return e;
     if (path == 0 && patch_wanted(a))
         e = launch_conv_patch(a, stream, options().patch >= 0 ? options().patch_nf : 4, options().patch_pr, options().patch >= 0 ? options().patch_waves : 16,

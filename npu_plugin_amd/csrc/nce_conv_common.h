@@ -276,6 +276,17 @@ hipError_t launch_conv_tiled(const ConvArgs& a, hipStream_t stream, int shape, c
 // Split-reduction kernel for tasks with few output tiles: a workgroup's waves share out one tile's reduction. shape 1..5: see
 // nce_conv_split.hip.
 hipError_t launch_conv_split(const ConvArgs& a, hipStream_t stream, int shape, const FuseAdd* fuse = nullptr);
+// Band kernel for kernels larger than 1x1 over few input channels: weights slice and the input rows of a run of pixels in LDS.
+// shape 1 .. 4: runs of 128, 256, 384 or 576 pixels.
+hipError_t launch_conv_band(const ConvArgs& a, hipStream_t stream, int shape);
+// The band kernel's plan for a task and shape (ok = false: the rows do not fit): channel fragments per slice, runs of a
+// workgroup, workgroups, fetch passes of its first run and of every further one.
+struct BandShape {
+    bool ok;
+    int nf;
+    int64_t tpg, groups, first_passes, fresh_passes;
+};
+BandShape band_shape_for(const ConvArgs& a, int shape);
 // Patch kernel for kernels larger than 1x1 at stride 1: weights slice and the patch's input pixels (with halo) both in LDS.
 // nf = 0 / pr = 0 / waves = 0: automatic channel fragments per slice (2 or 4) / output rows per patch / waves per workgroup (8, 16);
 // npx = 1 (with 16 waves): one pixel fragment per wave and group instead of two.
