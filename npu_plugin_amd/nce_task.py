@@ -17,6 +17,15 @@ import ctypes as C
 from . import _abi as abi
 from ._abi import *  # noqa: F401,F403  (re-export the enums)
 
+try:
+    from ._native import EnqueueBase
+except ImportError as _missing:  # (not built yet: the package can be imported, an Executor cannot be created)
+    _missing_native = str(_missing)
+
+    class EnqueueBase:
+        def _bind(self, *args):
+            raise RuntimeError(f"npu_plugin_amd/_native.so is missing: build the library first (make -C npu_plugin_amd/csrc): {_missing_native}")
+
 
 class NCEError(RuntimeError):
     def __init__(self, code, log=""):
@@ -106,7 +115,7 @@ class NCEClusterTask:
         self.desc.kernel_pad_top, self.desc.kernel_pad_bottom = top, bottom
         self._variants = []
         self._ppe = None
-        self._wired = (None, None, None)  # (descriptor, variant, PPE task) that finalize() has connected
+        self._wired = (None, None, None, 0)  # (descriptor, variant, PPE task) that finalize() has connected, the first's address
 
     def addDPUTask(self, outStart, outEnd, pad=(0, 0, 0, 0), mpeMode=abi.MPE_CUBOID_16x16, clusterId=0):
         """outStart / outEnd: [x, y, z] inclusive; pad: (left, right, top, bottom)
@@ -163,11 +172,11 @@ class NCEClusterTask:
             if wired[0] is desc and wired[1] is variants[0] and wired[2] is ppe and desc.num_variants == 1:
                 return desc
             desc.variants = C.pointer(variants[0])
-            self._wired = (desc, variants[0], ppe)
+            self._wired = (desc, variants[0], ppe, C.addressof(desc))
         else:
             self._variant_array = (abi.DpuTask * max(n, 1))(*variants)
             desc.variants = C.cast(self._variant_array, C.POINTER(abi.DpuTask)) if n else None
-            self._wired = (None, None, None)
+            self._wired = (None, None, None, 0)
         desc.num_variants = n
         desc.ppe = C.pointer(ppe) if ppe is not None else None
         return desc
@@ -201,7 +210,7 @@ class TaskList:
             self._h = C.c_void_p()
 
 
-class Executor:
+class Executor(EnqueueBase):
     """nceExecutorCreate / Enqueue / Synchronize. device_id < 0 gives a validate-only executor."""
 
     def __init__(self, device_id=0, log_level=2):
@@ -212,6 +221,7 @@ class Executor:
         rc = self._lib.nceExecutorCreate(abi.ExecutorDesc(device_id, log_level), C.byref(self._h), C.byref(self._log))
         if rc != abi.SUCCESS:
             raise NCEError(rc, f"nceExecutorCreate(device_id={device_id}) failed; a GPU is required, there is no CPU fallback")
+        self._bind(C.cast(self._task_enqueue, C.c_void_p).value, self._h.value or 0)
 
     def log(self):
         size = C.c_size_t(0)
@@ -230,7 +240,9 @@ class Executor:
     def validate(self, task):
         self._check(self.validate_code(task))
 
-    def enqueue(self, task, stream=None):
+    # enqueue(task, stream=None) is EnqueueBase's (csrc/nce_pyenqueue.cpp): it calls the library straight away when the task's
+    # descriptor is wired as finalize() would leave it, and this otherwise.
+    def _enqueue_slow(self, task, stream):
         rc = self._task_enqueue(self._h, C.addressof(task.finalize()), stream)
         if rc != abi.SUCCESS:
             self._check(rc)
@@ -243,6 +255,7 @@ class Executor:
 
     def destroy(self):
         if self._h:
+            self._bind(0, 0)
             self._lib.nceExecutorDestroy(self._h)
             self._h = C.c_void_p()
 
