@@ -96,6 +96,7 @@ nce::Options read_options() {
     if (const char* e = getenv("NCE_HIP_CONV_TILE")) o.halo_tile = atoi(e);
     if (const char* e = getenv("NCE_HIP_CONV_TILED")) o.tiled = atoi(e);
     if (const char* e = getenv("NCE_HIP_CONV_BAND")) o.band = atoi(e);
+    if (const char* e = getenv("NCE_HIP_WINDOW_MFMA")) o.window = atoi(e);
     if (const char* e = getenv("NCE_HIP_CONV_SPLIT")) o.split = atoi(e);
     if (const char* e = getenv("NCE_HIP_CONV_PATCH")) {
         int nf = 0, pr = 0, wv = 0, npx = 0;

@@ -169,6 +169,7 @@ struct Options {
     int persistent_wait_us = 2000000;  // NCE_HIP_PERSISTENT_WAIT_US: time after which a persistent launch's waits give up
     int tiled = -1;           // NCE_HIP_CONV_TILED: -1 automatic, 0 never, 1.. force that shape of the LDS-tiled kernel
     int band = -1;            // NCE_HIP_CONV_BAND: -1 automatic, 0 never, 1 .. 4: that run length of the band kernel
+    int window = -1;          // NCE_HIP_WINDOW_MFMA: depthwise and average pool on the matrix cores: -1 automatic, 0 never, 1 wherever supported
     int split = -1;           // NCE_HIP_CONV_SPLIT: -1 automatic, 0 never, 1.. force that tile of the split-reduction kernel
     int patch = -1;           // NCE_HIP_CONV_PATCH: -1 automatic, 0 never, 1 = wherever its conditions hold; "nf,pr[,waves]" also forces its shape
     int patch_nf = 0, patch_pr = 0, patch_waves = 0, patch_npx = 0;
@@ -229,6 +230,8 @@ inline hipError_t replay(const RecordedLaunch& r, hipStream_t stream) {
 hipError_t launch_eltwise(const TaskDev& t, const Box& box, hipStream_t stream);
 hipError_t launch_pool(const TaskDev& t, const Box& box, bool is_max, hipStream_t stream);
 hipError_t launch_dwconv(const TaskDev& t, const Box& box, hipStream_t stream);
+// DWCONV / AVEPOOL on the matrix cores (nce_window_mfma.hip); hipErrorNotSupported when the window or its rows are beyond it.
+hipError_t launch_window_mfma(const TaskDev& t, const Box& box, bool depthwise, hipStream_t stream);
 hipError_t launch_conv(const TaskDev& t, const Box& box, hipStream_t stream);
 // The convolution `conv` and the ELTWISE task `add` that directly follows it in a task list as ONE launch, when the add
 // reads the convolution's output and everything else allows it; hipErrorNotSupported (nothing launched) otherwise.

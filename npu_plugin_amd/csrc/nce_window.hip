@@ -64,12 +64,12 @@ struct WinArgs {
     Box box;
     int64_t npix;
     int32_t items_per_thread;
+    int32_t slab_groups;  // channel groups of a slab (the last one may have fewer)
     uint32_t nblocks;  // item blocks per channel slab (the grid is padded to a multiple of the XCD count)
     uint32_t a_xor;   // 0x80808080 for i8 activations
     uint32_t fill;    // word of re-biased zero-point bytes for out-of-image taps
     int32_t zpu;      // zero point of the re-biased (unsigned) activation bytes
     // I32 kernels (item count and tensor strides below 2^31): divisors of the item decomposition
-    int32_t nslab_full;            // channel groups of every slab but the last
     FastDiv div_full, div_last;    // by the channel groups of a full slab / of the last slab
     FastDiv div_bw, div_bh;
 };
@@ -92,8 +92,8 @@ __global__ __launch_bounds__(NT) void window_kernel(WinArgs a) {
     const TaskDev& t = a.t;
     const Box& box = a.box;
     const int32_t cgroups = box.bc >> 4;
-    const int32_t slab0 = blockIdx.y * SLAB_GROUPS;
-    const int32_t nslab = min(SLAB_GROUPS, cgroups - slab0);
+    const int32_t slab0 = blockIdx.y * a.slab_groups;
+    const int32_t nslab = min(a.slab_groups, cgroups - slab0);
     const int ntaps = t.ky * t.kx;
     float* s_w = reinterpret_cast<float*>(smem);
 
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(NT) void window_kernel(WinArgs a) {
         int64_t n;
         if constexpr (I32) {
             const uint32_t u = (uint32_t)item;
-            const uint32_t r1 = fdiv(u, nslab == a.nslab_full ? a.div_full : a.div_last);
+            const uint32_t r1 = fdiv(u, nslab == a.slab_groups ? a.div_full : a.div_last);
             cg = (int32_t)(u - r1 * (uint32_t)nslab);
             const uint32_t r2 = fdiv(r1, a.div_bw);
             bx = (int32_t)(r1 - r2 * (uint32_t)box.bw);
@@ -537,8 +537,13 @@ hipError_t launch_window_kk(const TaskDev& t, const Box& box, hipStream_t s) {
     a.npix = (int64_t)t.out.n * box.bh * box.bw;
     const int32_t cgroups = box.bc >> 4;
     if (a.npix == 0 || cgroups == 0) return hipSuccess;
-    const int nslabs = (cgroups + SLAB_GROUPS - 1) / SLAB_GROUPS;
-    const int64_t items = a.npix * (cgroups < SLAB_GROUPS ? cgroups : SLAB_GROUPS);
+    // Slabs of eight groups read whole 128-byte lines; but 9 groups as 8 + 1 leave a slab whose lanes all read 16 bytes of
+    // different pixels (3x3 average pool of 36 x 97 x 97 x 144 at stride 2: 59 us, 21 us as 5 + 4; 5x5 depthwise over 784
+    // channels, 35 x 86 x 86, stride 2: 196 -> 150 us). Equal slabs where the last one would be less than half full or there are two
+    // (8 + 5 -> 7 + 6: 13.4 -> 10.7 us); not for 8 + 8 + 8 + 4, which then read parts of lines (129 -> 160 us).
+    const int nslabs = (cgroups + SLAB_GROUPS - 1) / SLAB_GROUPS, rest = cgroups % SLAB_GROUPS;
+    a.slab_groups = rest == 0 || (rest >= 4 && nslabs > 2) ? SLAB_GROUPS : (cgroups + nslabs - 1) / nslabs;
+    const int64_t items = a.npix * a.slab_groups;
     // (several items per thread amortise the per-workgroup constants of large tasks; max pool has none and measured
     // fastest with one item per thread at every size)
     a.items_per_thread = (MODE != MODE_MAX && items > (int64_t)NT * 8192) ? 4 : 1;
@@ -549,10 +554,8 @@ hipError_t launch_window_kk(const TaskDev& t, const Box& box, hipStream_t s) {
     a.zpu = t.in.zp + (t.in.is_signed ? 128 : 0);
     a.fill = (uint32_t)a.zpu * 0x01010101u;
     const size_t lds = MODE == MODE_DW ? (size_t)t.ky * t.kx * SLAB_CH * sizeof(float) : 0;
-    const int32_t full = cgroups < SLAB_GROUPS ? cgroups : SLAB_GROUPS;
-    a.nslab_full = full;
-    a.div_full = make_fastdiv((uint32_t)full);
-    a.div_last = make_fastdiv((uint32_t)(cgroups - (nslabs - 1) * SLAB_GROUPS));
+    a.div_full = make_fastdiv((uint32_t)a.slab_groups);
+    a.div_last = make_fastdiv((uint32_t)(cgroups - (nslabs - 1) * a.slab_groups));
     a.div_bw = make_fastdiv((uint32_t)box.bw);
     a.div_bh = make_fastdiv((uint32_t)box.bh);
     bool i32 = blocks * NT * a.items_per_thread < 0x7fffffffLL;
@@ -561,8 +564,24 @@ hipError_t launch_window_kk(const TaskDev& t, const Box& box, hipStream_t s) {
     return launch_window_i32<MODE, KK, false>(a, blocks, nslabs, lds, s);
 }
 
+// Which depthwise convolutions and average pools take the matrix cores (nce_window_mfma.hip). Measured over 120 tasks: windows
+// of more than nine taps without a compile-time form in every case (7x7: 17 -> 9 us for small tasks, 78 -> 35 us for 32 x 24 x 24
+// x 832); 5x5 at stride 1 from about 4.5 million outputs on (level at 4 million, 16.7 -> 12.8 us at 5.3 million, 201 -> 110 us at 87 million). Behind it for 5x5 at
+// stride 2 (its rows hold two column planes and twice the pixels), 3x3 (memory-bound either way) and average pools, and its
+// 5.5-7 us for the smallest tasks are behind the 4-6 us of the kernel here.
+static bool mfma_wanted(const TaskDev& t, const Box& box, bool depthwise) {
+    if (options().window >= 0) return options().window > 0;
+    if (!depthwise) return false;
+    if (t.ky == 5 && t.kx == 5) return t.sx == 1 && t.sy == 1 && (int64_t)t.out.n * box.bh * box.bw * box.bc >= 4500000;
+    return t.ky * t.kx > 9;
+}
+
 template <int MODE>
 hipError_t launch_window(const TaskDev& t, const Box& box, hipStream_t s) {
+    if (MODE != MODE_MAX && mfma_wanted(t, box, MODE == MODE_DW)) {
+        const hipError_t e = launch_window_mfma(t, box, MODE == MODE_DW, s);
+        if (e != hipErrorNotSupported) return e;
+    }
     if (MODE == MODE_MAX) {
         // the compile-time windows of the max pool rely on every window of the box overlapping the image
         const bool reach = t.pt < t.ky && t.pl < t.kx && (int64_t)(box.y0 + box.bh - 1) * t.sy - t.pt <= t.in.h - 1 &&
