@@ -79,7 +79,6 @@ struct ScopedLaunch {
     ScopedLaunch(const nce::Options* opt, std::vector<nce::RecordedLaunch>* record, nce_log_s* log = nullptr) : saved(nce::tls_launch) {
         nce::tls_launch.opt = opt;
         nce::tls_launch.record = record;
-        nce::tls_launch.in_list = false;
         nce::tls_launch.log = log;
     }
     ~ScopedLaunch() { nce::tls_launch = saved; }
@@ -961,7 +960,6 @@ nce_result_t enqueue_list(nce_task_list_handle_t list, void* hip_stream, bool fi
             std::vector<PkAlt> alts;
             {
                 const ScopedLaunch ctx(&ex->opt, &list->launches, ex->log);
-                nce::tls_launch.in_list = list->plans.size() > 1;
                 const nce_result_t r = run_plans(ex, list->plans, nullptr, persistent ? &alts : nullptr);
                 if (r != NCE_RESULT_SUCCESS) {
                     list->launches.clear();

@@ -195,8 +195,6 @@ struct LaunchContext {
     // Per-XCD form: the task is one eighth of the batch, to be run by the 32 CUs of one XCD inside a persistent segment
     // (grids are sized for 32 CUs; only the weights-resident convolution kernels take part).
     bool per_xcd = false;
-    // The launch is one of a list of tasks: its weights were last read a whole pass ago and come from memory, not from L2.
-    bool in_list = false;
 };
 extern thread_local LaunchContext tls_launch;
 inline const Options& options() {

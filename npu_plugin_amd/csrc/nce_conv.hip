@@ -326,20 +326,23 @@ static bool patch_wanted(const ConvArgs& a) {
 // The split-reduction, LDS-tiled and weights-resident kernels serve overlapping ranges of tasks, and which of their tiles is
 // ahead depends on how the grid fills the chip: one rule of thumb per kernel left 30 % on the table. So each has a cost
 // estimate in microseconds - a few terms that count what the kernel does (rounds of workgroups, reduction steps per round,
-// bytes through a CU's load path, fragments exchanged, output bytes), with coefficients fitted by non-negative least squares
-// on the relative error over 734 measured tasks: random shapes, types and zero points, 1 to 64 images, and the ResNet-50
-// layers at batch 1 to 128, every kernel and tile forced on every task. The estimates are within 10-25 % of the measured
-// times for nine tasks in ten; the kernel chosen by them is on average 3 % slower than the best one of each task, where the
-// patch and weights-resident kernels and their fallbacks alone were 39 % slower.
-static double estimate_split(const ConvArgs& a, int shape) {
+// bytes through a CU's load path, fragments exchanged, output bytes, a fused add's bytes), with coefficients fitted by
+// non-negative least squares on the relative error over 685 tasks enqueued alone (random shapes, types and zero points, 1 to 64
+// images, and the ResNet-50 layers at batch 1 to 128) and the layers of eleven ResNet-50 graphs (2 to 128 images, 129 to 224
+// pixels wide: cold weights, fused adds), every kernel and tile forced on every one. The kernel chosen is on average 2.5 % slower
+// than the best one of a task alone and 2.0 % of a layer in its graph; a fit to tasks alone, with batches of powers of two only,
+// was 4.1 and 4.3 % (and 7 % for the graph of 96 images: 1394 -> 1322 us).
+static double estimate_split(const ConvArgs& a, int shape, double added) {
     struct Tile {
         int nf, bf, depth;
-        double base, round, kib, frags, step, wait;
+        double base, round, kib, frags, step, wait, add;
     };
     static const Tile tiles[5] = {
-        {1, 1, 8, 3.27, 1.521, 0.01781, 0.0444, 0.0, 0.0},     {2, 1, 5, 3.41, 2.029, 0.0, 0.0478, 0.2985, 0.0},
-        {2, 2, 4, 3.67, 1.528, 0.0129, 0.1141, 0.0, 0.0},      {4, 2, 3, 4.07, 2.238, 0.0, 0.1135, 0.3513, 0.4308},
-        {4, 4, 2, 4.96, 2.413, 0.0, 0.1274, 0.0894, 1.213},
+        {1, 1, 8, 3.179, 1.555, 0.01888, 0.02927, 0.0, 0.0, 1.072},
+        {2, 1, 5, 3.483, 2.022, 0.00418, 0.03755, 0.2124, 0.0, 0.3626},
+        {2, 2, 4, 3.677, 1.518, 0.0142, 0.1007, 0.0, 0.0, 0.7448},
+        {4, 2, 3, 4.234, 2.212, 0.0, 0.1093, 0.53, 0.0, 0.5636},
+        {4, 4, 2, 5.13, 2.269, 0.0, 0.1179, 0.2718, 0.9225, 0.638},
     };
     const Tile& t = tiles[shape - 1];
     const int64_t slices = (a.KG + 3) / 4;
@@ -350,22 +353,22 @@ static double estimate_split(const ConvArgs& a, int shape) {
     const int64_t resident = std::max<int64_t>(1, std::min<int64_t>(156 / (waves * std::max(t.depth * f, slots)), 32 / waves));
     const double rounds = (double)((groups + 256 * resident - 1) / (256 * resident)), per_cu = (double)((groups + 255) / 256);
     return t.base + t.round * (rounds - 1) + t.kib * per_cu * (double)(slices * f) + t.frags * per_cu * (t.nf * t.bf) +
-           t.step * rounds * (double)per_wave + t.wait * rounds * (double)((per_wave + t.depth - 1) / t.depth);
+           t.step * rounds * (double)per_wave + t.wait * rounds * (double)((per_wave + t.depth - 1) / t.depth) + t.add * added;
 }
 
-static double estimate_tiled(const ConvArgs& a, int shape) {
+static double estimate_tiled(const ConvArgs& a, int shape, double added) {
     struct Tile {
         int bm, bn, resident;
-        double base, step, more, round, group, unit, unit_alone, wsum, asum, out;
+        double base, step, more, round, group, unit, unit_alone, wsum, asum, out, flow, add;
     };
     static const Tile tiles[7] = {
-        {256, 256, 1, 2.113, 1.283, 1.559, 0.0, 5.08, 0.2087, 0.0, 0.2207, 1.845, 0.1322},
-        {256, 128, 1, 1.725, 0.7668, 0.8765, 4.016, 0.0, 0.1812, 0.0, 0.1575, 0.2475, 0.1272},
-        {128, 128, 2, 2.285, 0.4806, 0.332, 1.303, 1.013, 0.1278, 0.0, 0.1621, 0.1994, 0.1388},
-        {128, 64, 3, 1.796, 0.4204, 0.1802, 1.995, 0.5824, 0.0729, 0.0622, 0.1033, 0.0841, 0.0462},
-        {64, 128, 3, 0.912, 0.3846, 0.18, 2.411, 0.747, 0.0898, 0.0603, 0.1252, 0.0854, 0.0439},
-        {64, 64, 4, 1.909, 0.3144, 0.1124, 1.63, 0.3388, 0.0618, 0.0767, 0.0697, 0.0372, 0.0713},
-        {256, 64, 1, 1.443, 0.6594, 0.6942, 3.968, 0.0, 0.1804, 0.0, 0.1785, 0.1292, 0.1069},
+        {256, 256, 1, 2.229, 1.342, 1.432, 5.275, 0.0, 0.1138, 0.0, 0.1747, 2.033, 0.07449, 0.2299, 0.4591},
+        {256, 128, 1, 1.887, 0.7743, 0.831, 3.978, 0.0, 0.1562, 0.0, 0.1094, 0.2146, 0.08869, 0.1359, 0.3483},
+        {128, 128, 2, 1.859, 0.5219, 0.3105, 2.025, 0.8085, 0.08485, 0.0, 0.1121, 0.1843, 0.0818, 0.09549, 0.2443},
+        {128, 64, 3, 1.954, 0.4576, 0.1686, 1.94, 0.4668, 0.09575, 0.0, 0.07982, 0.0638, 0.1026, 0.02258, 0.2577},
+        {64, 128, 3, 1.845, 0.4292, 0.1603, 1.262, 0.9446, 0.1032, 0.0, 0.07895, 0.07496, 0.1149, 0.02828, 0.2633},
+        {64, 64, 4, 1.712, 0.3593, 0.07846, 1.915, 0.2991, 0.07781, 0.0006697, 0.04486, 0.02911, 0.05387, 0.03719, 0.2377},
+        {256, 64, 1, 1.721, 0.6708, 0.7002, 0.0, 3.769, 0.1713, 0.0, 0.1426, 0.103, 0.116, 0.03162, 0.3442},
     };
     const Tile& t = tiles[shape - 1];
     const double steps = (double)((a.KG + 7) / 8);
@@ -374,20 +377,25 @@ static double estimate_tiled(const ConvArgs& a, int shape) {
     const bool units = a.IC % 128 != 0 || a.dw != 0;
     return t.base + t.step * steps + t.more * steps * (per_cu - 1) + t.round * rounds + t.group * per_cu +
            (units ? t.unit * steps * per_cu + t.unit_alone * steps : 0.0) + (a.da != 0 ? t.wsum * steps * per_cu : 0.0) +
-           (a.dw != 0 ? t.asum * steps * per_cu : 0.0) + 1e-6 * t.out * (double)a.M * a.bc;
+           (a.dw != 0 ? t.asum * steps * per_cu : 0.0) + 1e-6 * t.out * (double)a.M * a.bc +
+           t.flow * steps * (double)groups / 256.0 + t.add * added;
 }
 
-static double estimate_wres(const ConvArgs& a, const WresShape& s) {
+static double estimate_wres(const ConvArgs& a, const WresShape& s, double added) {
     const double steps = (double)((a.KG + 3) / 4), rounds = (double)((s.groups * s.slices + 255) / 256);
     const double tiles = (double)((s.tiles_per_group + 7) / 8);  // per wave
     const double out = 1e-6 * (double)a.M * a.bc, in = 1e-6 * (double)a.M * a.SY * a.SX * a.IC * (double)s.slices;
     const double stage = steps * s.nf * rounds, mma = tiles * steps * s.nf * s.bf * rounds, sums = a.da != 0 || a.dw != 0 ? stage : 0.0;
     const double asums = a.dw != 0 ? tiles * steps * s.bf * rounds : 0.0;
-    if (a.IC % 64 != 0)  // (per-lane loads)
-        return 3.421 * rounds + 0.00143 * stage + 0.00775 * mma + 0.1003 * tiles * rounds + 0.1024 * tiles * steps * s.bf * rounds + 0.00868 * sums +
-               0.02104 * asums + 0.4475 * out + 0.0232 * in;
-    return 3.21 + 0.00669 * stage + 0.0859 * tiles * steps * rounds + 0.02955 * mma + 0.0119 * sums + 0.01219 * asums + 0.2285 * out + 0.0016 * in +
-           (a.bc % 64 != 0 ? 0.2556 * out : 0.0);
+    if (a.IC % 64 != 0)  // (per-lane loads; the taps of the largest windows find their lines in L1 while few slices share it)
+        return (a.KY * a.KX > 25 && s.slices <= 4 ? 0.8 : 1.0) *
+               (3.37 * rounds + 0.007261 * mma + 0.1355 * tiles * rounds + 0.1195 * tiles * steps * s.bf * rounds + 0.002633 * sums + 0.01683 * asums +
+                0.3096 * out + 0.02463 * in);
+    // (inputs beyond 40 MB: every slice reads them again, and the caches behind the L2s no longer hold them for it)
+    const double far = std::max(0.0, 1e-6 * (double)a.M * (a.KY * a.KX == 1 ? 1 : a.SY * a.SX) * a.IC - 40.0) * (double)s.slices;
+    const double waste = 1e-6 * (double)a.M * (double)(s.slices * 16 * s.nf - a.bc);  // outputs of channels past the last one
+    return 3.591 + 0.0193 * stage + 0.0574 * tiles * steps * rounds + 0.0285 * mma + 0.0011 * sums + 0.05 * asums + 0.2311 * out + 0.0047 * in +
+           0.8 * waste + 0.127 * far + 0.3552 * added;
 }
 
 // (fitted the same way on 272 tasks with kernels larger than 1x1 over ragged channel counts, 1 to 128 images, every run length
@@ -421,20 +429,16 @@ static ConvChoice choose_conv(const ConvArgs& a, bool fused) {
     if (options().band > 0) return {0, 0, options().band};
     ConvChoice c = {0, 0, 0};
     const WresShape s = wres_shape_for(a, fused);
-    // (The weights-resident kernel's estimate is the least certain: it has to be beaten by 10 %. Of the 734 tasks four then come
-    // out more than 4 % slower than it. Those were tasks enqueued again and again, whose weights sit in L2. In a list they come
-    // from memory, a launch of any kernel is slower than its estimate - and the LDS-tiled kernel, which requests them all
-    // ahead, by less: ResNet-50 at batch 32, 663 us with the factor for single tasks, 651 with the one for lists.)
-    const double wres_factor = tls_launch.in_list ? 1.0 : 0.9;
+    const double added = fused ? 1e-6 * (double)a.M * a.bc : 0.0;  // megabytes of the residual add's operand and of its result
     // (what is neither a weights-resident nor a patch task would take a kernel that gathers or re-stages its operands: those
     // are never ahead)
-    double best = !fused && patch_wanted(a) ? 0.0 : s.ok && (!fused || s.nf == 4) ? wres_factor * estimate_wres(a, s) : 1e30;
+    double best = !fused && patch_wanted(a) ? 0.0 : s.ok && (!fused || s.nf == 4) ? estimate_wres(a, s, added) : 1e30;
     if (options().split < 0)
         for (int i = 1; i <= 5; ++i)
-            if (const double t = estimate_split(a, i); t < best) best = t, c = {i, 0, 0};
+            if (const double t = estimate_split(a, i, added); t < best) best = t, c = {i, 0, 0};
     if (options().tiled < 0 && !(fused && (a.IC % 128 != 0 || a.dw != 0)))
         for (int i = fused ? 2 : 1; i <= 7; ++i)  // (256 x 256 tiles, one workgroup per CU, leave an add's traffic with nothing beside it)
-            if (const double t = estimate_tiled(a, i); t < best) best = t, c = {0, i, 0};
+            if (const double t = estimate_tiled(a, i, added); t < best) best = t, c = {0, i, 0};
     // (a 1x1 kernel has no rows to share between taps; whole 64-channel pixels are read as they are by the kernels above)
     if (options().band < 0 && !fused && a.KY * a.KX > 1 && a.IC % 64 != 0)
         for (int i = 1; i <= 4; ++i)
